@@ -34,7 +34,8 @@ using namespace fe_sparse;
 struct PcgState {
   double alpha, beta, gamma, gamma_prev;
   double rr, rr_ref, rr_true, bb;
-  double tol2bb, ru_delta2, rr_best, pad0;
+  double tol2bb, ru_delta2, rr_best;
+  double rgamma, ralpha;  // reciprocals of gamma and alpha, formed off the next sums' critical path
   int32_t iter, max_iter;
   int32_t done;     // 0 running, 1 converged, 2 iteration limit / stagnation, 3 breakdown
   int32_t need_ru;  // 1: reliable update / true-residual check requested
@@ -309,46 +310,38 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(const Tile* __restrict__ til
     for (int k = 0; k < 3; ++k) partials[(int64_t)k * ntiles + tid_] = v[k];
 }
 
-// One workgroup per segment: the Chronopoulos-Gear scalars for the next iteration.
+// What the scalars of the next iteration are formed from, beside the sums (read ahead of them).
+struct CgIn {
+  double gamma, rgamma, ralpha, tol2bb, ru_delta2, rr_ref;
+  int32_t iter, max_iter, mixed, ru_pending;
+};
+__device__ inline CgIn cg_in(const PcgState* s) {
+  return CgIn{s->gamma, s->rgamma, s->ralpha, s->tol2bb, s->ru_delta2, s->rr_ref,
+              s->iter + 1, s->max_iter, s->mixed, s->ru_pending};
+}
+
+// The Chronopoulos-Gear scalars for the next iteration from the sums v = (r.u, w.u, r.r), by one thread.
 // last: this is the chunk's last iteration (a pending reliable update is requested now).
-__global__ __launch_bounds__(kRed) void k_cg_reduce(const int32_t* __restrict__ seg_tiles, int ntiles,
-                                                    const double* __restrict__ partials,
-                                                    PcgState* st, int last) {
-  PcgState* s = st + blockIdx.x;
-  // the tile range, the running test and the fields the update reads are loaded together (only
-  // thread 0 writes the state, after the sums); the test is uniform
-  const int t0 = seg_tiles[blockIdx.x], t1 = seg_tiles[blockIdx.x + 1];
-  const int32_t done = s->done, need_ru = s->need_ru;
-  const double gamma0 = s->gamma, alpha0 = s->alpha, tol2bb = s->tol2bb;
-  const double ru_delta2 = s->ru_delta2, rr_ref = s->rr_ref;
-  const int32_t iter = s->iter + 1, max_iter = s->max_iter, mixed = s->mixed;
-  int32_t ru_pending = s->ru_pending;
-  // an empty asm that takes the values keeps their loads ahead of the exit (the compiler would
-  // otherwise sink each one to its first use, a memory round trip apiece)
-  asm volatile("" ::"s"(t0), "s"(t1), "s"(gamma0), "s"(alpha0), "s"(tol2bb), "s"(ru_delta2), "s"(rr_ref),
-               "s"(iter), "s"(max_iter), "s"(mixed), "s"(ru_pending), "s"(ntiles), "s"(partials));
-  if (done | need_ru) return;
-  double v[3];
-  seg_sum<3>(partials, ntiles, t0, t1, v);
-  if (threadIdx.x != 0) return;
+__device__ inline void cg_scalars(PcgState* s, const CgIn& c, const double (&v)[3], int last) {
   const double g = v[0], dl = v[1];
-  s->iter = iter;
+  s->iter = c.iter;
   s->rr = v[2];
   if (!isfinite(g) || !isfinite(dl) || !isfinite(v[2]) || g < 0.0) {
     s->done = 3;
     return;
   }
-  s->gamma_prev = gamma0;
+  s->gamma_prev = c.gamma;
   s->gamma = g;
   // convergence claims and the iteration limit hand over to the true-residual check at the end of
   // the chunk; (mixed precision) the reliable-update threshold marks the update pending
-  if (v[2] <= tol2bb || iter >= max_iter) {
+  if (v[2] <= c.tol2bb || c.iter >= c.max_iter) {
     s->need_ru = 1;
     return;
   }
-  if (mixed && v[2] < ru_delta2 * rr_ref) s->ru_pending = ru_pending = 1;
-  const double beta = g / gamma0;
-  const double den = dl - beta * g / alpha0;
+  const bool pending = c.ru_pending || (c.mixed && v[2] < c.ru_delta2 * c.rr_ref);
+  if (pending) s->ru_pending = 1;
+  const double beta = g * c.rgamma;
+  const double den = dl - beta * g * c.ralpha;
   if (!(den > 0.0)) {
     // the recurrences lost positivity (rounding, most often in FP32): restart from the true
     // residual; a genuine breakdown shows up there as p.Ap <= 0
@@ -359,8 +352,31 @@ __global__ __launch_bounds__(kRed) void k_cg_reduce(const int32_t* __restrict__ 
   }
   s->beta = beta;
   s->alpha = g / den;
+  s->rgamma = 1.0 / g;
+  s->ralpha = den / g;
   // the update replaces r, u, w, s and recomputes beta and alpha from gamma_prev, as at a hand-over
-  if (last && ru_pending) s->need_ru = 1;
+  if (last && pending) s->need_ru = 1;
+}
+
+// One workgroup per segment: the sums over its tiles, then the scalars.
+__global__ __launch_bounds__(kRed) void k_cg_reduce(const int32_t* __restrict__ seg_tiles, int ntiles,
+                                                    const double* __restrict__ partials,
+                                                    PcgState* st, int last) {
+  PcgState* s = st + blockIdx.x;
+  // the tile range, the running test and the fields the update reads are loaded together (only
+  // thread 0 writes the state, after the sums); the test is uniform
+  const int t0 = seg_tiles[blockIdx.x], t1 = seg_tiles[blockIdx.x + 1];
+  const int32_t done = s->done, need_ru = s->need_ru;
+  const CgIn c = cg_in(s);
+  // an empty asm that takes the values keeps their loads ahead of the exit (the compiler would
+  // otherwise sink each one to its first use, a memory round trip apiece)
+  asm volatile("" ::"s"(t0), "s"(t1), "s"(c.gamma), "s"(c.rgamma), "s"(c.ralpha), "s"(c.tol2bb), "s"(c.ru_delta2),
+               "s"(c.rr_ref), "s"(c.iter), "s"(c.max_iter), "s"(c.mixed), "s"(c.ru_pending), "s"(ntiles), "s"(partials));
+  if (done | need_ru) return;
+  double v[3];
+  seg_sum<3>(partials, ntiles, t0, t1, v);
+  if (threadIdx.x != 0) return;
+  cg_scalars(s, c, v, last);
 }
 
 // --------------------------------------------------------------------------------------------------
@@ -398,6 +414,34 @@ __global__ __launch_bounds__(kBlock) void k_ru_residual(const Tile* __restrict__
   if (threadIdx.x == 0) partials[tid_] = v[0];
 }
 
+// Part 2's decision from the true residual's square rr, by one thread.
+__device__ inline void ru_decide(PcgState* s, double rr) {
+  s->rr_true = rr;
+  if (rr <= s->tol2bb) {
+    s->done = 1;
+  } else if (s->iter >= s->max_iter) {
+    s->done = 2;
+  } else {
+    if (rr < 0.81 * s->rr_best) {
+      s->rr_best = rr;
+      s->stall = 0;
+    } else if (++s->stall >= kStallLimit) {
+      s->done = 2;
+    }
+    // the recursive residual drifted far below the true one: the direction is stale, restart
+    if (!s->first && rr > 4.0 * s->rr) {
+      s->first = 1;
+      s->restarts += 1;
+    }
+    if (s->restarts > (s->mixed ? kMaxRestarts32 : kMaxRestarts64)) s->done = 2;
+  }
+  if (s->done) {
+    s->rr = rr;
+    s->n_ru += 1;
+    s->need_ru = 0;
+  }
+}
+
 // Part 2 (per segment): judge the true residual -- converged, out of iterations, stagnating, or
 // continue with the replaced residual (restarting the direction when it drifted).
 __global__ __launch_bounds__(kRed) void k_ru_decide(const int32_t* __restrict__ seg_tiles, int ntiles,
@@ -408,31 +452,7 @@ __global__ __launch_bounds__(kRed) void k_ru_decide(const int32_t* __restrict__ 
   if (!seg_updating(s)) return;
   double v[1];
   seg_sum<1>(partials, ntiles, t0, t1, v);
-  if (threadIdx.x != 0) return;
-  s->rr_true = v[0];
-  if (v[0] <= s->tol2bb) {
-    s->done = 1;
-  } else if (s->iter >= s->max_iter) {
-    s->done = 2;
-  } else {
-    if (v[0] < 0.81 * s->rr_best) {
-      s->rr_best = v[0];
-      s->stall = 0;
-    } else if (++s->stall >= kStallLimit) {
-      s->done = 2;
-    }
-    // the recursive residual drifted far below the true one: the direction is stale, restart
-    if (!s->first && v[0] > 4.0 * s->rr) {
-      s->first = 1;
-      s->restarts += 1;
-    }
-    if (s->restarts > (s->mixed ? kMaxRestarts32 : kMaxRestarts64)) s->done = 2;
-  }
-  if (s->done) {
-    s->rr = v[0];
-    s->n_ru += 1;
-    s->need_ru = 0;
-  }
+  if (threadIdx.x == 0) ru_decide(s, v[0]);
 }
 
 // Part 3 (tiles): r = r64, u = M r (and p, s cleared on a (re)start).
@@ -516,12 +536,10 @@ __global__ __launch_bounds__(kBlock) void k_ru_spmv(const Tile* __restrict__ til
         }
     }
 #pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1)
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        au[d] += __shfl_xor(au[d], off, G);
-        ap[d] += __shfl_xor(ap[d], off, G);
-      }
+    for (int d = 0; d < D; ++d) {
+      au[d] = group_sum<G>(au[d]);
+      ap[d] = group_sum<G>(ap[d]);
+    }
     if (lane < D) {
       const int64_t k = i * D + lane;
       const T wk = pick<T, D>(au, lane), sk = pick<T, D>(ap, lane);
@@ -541,17 +559,8 @@ __global__ __launch_bounds__(kBlock) void k_ru_spmv(const Tile* __restrict__ til
     for (int k = 0; k < 5; ++k) partials[(int64_t)k * ntiles + tid_] = acc5[k];
 }
 
-// Part 5 (per segment): beta = gamma/gamma_prev (0 on a (re)start) and the exact alpha of the
-// direction p' = u + beta p: p'.Ap' = (u,w) + 2 beta (u,s) + beta^2 (p,s).
-__global__ __launch_bounds__(kRed) void k_ru_finish(const int32_t* __restrict__ seg_tiles, int ntiles,
-                                                    const double* __restrict__ partials,
-                                                    PcgState* st) {
-  PcgState* s = st + blockIdx.x;
-  const int t0 = seg_tiles[blockIdx.x], t1 = seg_tiles[blockIdx.x + 1];
-  if (!seg_updating(s)) return;
-  double v[5];
-  seg_sum<5>(partials, ntiles, t0, t1, v);
-  if (threadIdx.x != 0) return;
+// Part 5's scalars from the sums v = ((r,u), (u,w), (u,s), (p,s), (r,r)), by one thread.
+__device__ inline void ru_finish(PcgState* s, const double (&v)[5]) {
   const double g = v[0];
   if (!isfinite(g) || g < 0.0 || !isfinite(v[1])) {
     s->done = 3;
@@ -567,12 +576,27 @@ __global__ __launch_bounds__(kRed) void k_ru_finish(const int32_t* __restrict__ 
   s->beta = beta;
   s->alpha = g / pap;
   s->gamma = g;
+  s->rgamma = 1.0 / g;
+  s->ralpha = pap / g;
   s->first = 0;
   s->rr = v[4];
   s->rr_ref = s->rr_true;
   s->n_ru += 1;
   s->need_ru = 0;
   s->ru_pending = 0;
+}
+
+// Part 5 (per segment): beta = gamma/gamma_prev (0 on a (re)start) and the exact alpha of the
+// direction p' = u + beta p: p'.Ap' = (u,w) + 2 beta (u,s) + beta^2 (p,s).
+__global__ __launch_bounds__(kRed) void k_ru_finish(const int32_t* __restrict__ seg_tiles, int ntiles,
+                                                    const double* __restrict__ partials,
+                                                    PcgState* st) {
+  PcgState* s = st + blockIdx.x;
+  const int t0 = seg_tiles[blockIdx.x], t1 = seg_tiles[blockIdx.x + 1];
+  if (!seg_updating(s)) return;
+  double v[5];
+  seg_sum<5>(partials, ntiles, t0, t1, v);
+  if (threadIdx.x == 0) ru_finish(s, v);
 }
 
 // --------------------------------------------------------------------------------------------------
@@ -610,6 +634,8 @@ __global__ __launch_bounds__(kRed) void k_pcg_init(const int32_t* __restrict__ s
   s->alpha = 1.0;
   s->gamma = 1.0;
   s->gamma_prev = 1.0;
+  s->rgamma = 1.0;
+  s->ralpha = 1.0;
   s->rr_best = 1.0e308;
 }
 
@@ -668,6 +694,12 @@ __global__ void k_pcg_export(int nseg, const PcgState* st, fe_pcg_seg_stats* out
   out[g] = o;
 }
 
+}  // namespace
+
+#include "fe_pcg_team.h"
+
+namespace {
+
 // --------------------------------------------------------------------------------------------------
 // host side
 // --------------------------------------------------------------------------------------------------
@@ -680,6 +712,9 @@ struct Work {
   int32_t* seg_tiles;
   Tile* tiles;
   double* partials;
+  uint64_t* flags;  // the team's arrival flags, then its abort word
+  uint64_t* ut;     // its messages: u, and the partial dots
+  uint64_t* pt;
   fe_pcg_seg_stats* seg_stats;
   void* r;
   void* u;
@@ -713,7 +748,11 @@ Work layout_work(char* base, int64_t nb, int dof, int elem, int nseg, int64_t nt
   w.status = (PcgStatus*)take(sizeof(PcgStatus));
   w.seg_tiles = (int32_t*)take((nseg + 1) * (int64_t)sizeof(int32_t));
   w.tiles = (Tile*)take(std::max<int64_t>(1, ntiles) * (int64_t)sizeof(Tile));
-  w.partials = (double*)take(5 * std::max<int64_t>(1, ntiles) * (int64_t)sizeof(double));
+  w.partials = (double*)take(10 * std::max<int64_t>(1, ntiles) * (int64_t)sizeof(double));
+  const bool team = nseg == 1 && ntiles <= kTeamMaxTiles;
+  w.flags = (uint64_t*)take((kTeamMaxTiles + 1) * (int64_t)sizeof(uint64_t));
+  w.ut = (uint64_t*)take(team ? n * 2 * (int64_t)sizeof(uint64_t) : 0);
+  w.pt = (uint64_t*)take(team ? 12 * kTeamCopies * std::max<int64_t>(1, ntiles) * (int64_t)sizeof(uint64_t) : 0);
   w.seg_stats = (fe_pcg_seg_stats*)take(nseg * (int64_t)sizeof(fe_pcg_seg_stats));
   w.r = take(n * elem);
   w.u = take(n * elem);
@@ -739,6 +778,112 @@ struct Problem {
   const void* Ainv;
 };
 
+inline int chunk_of(const fe_pcg_opts* o) { return o->check_every > 0 ? o->check_every : 16; }
+inline int64_t max_chunks_of(const fe_pcg_opts* o) {
+  return 4 * ((int64_t)o->max_iter / chunk_of(o) + 2) + 8;
+}
+
+// Export the segments' statistics and read the aggregate status back (one synchronisation); flag: an extra
+// device word to read with it, or null.
+int finish_pcg(fe_handle* h, const Work& w, int nseg, fe_pcg_stats* s, const int32_t* flag, int32_t* flag_out) {
+  hipStream_t st = h->stream;
+  PcgStatus* pinned = (PcgStatus*)h->pinned;
+  hipLaunchKernelGGL(k_pcg_export, dim3((unsigned)ceil_div(nseg, 256)), dim3(256), 0, st, nseg, w.st,
+                     w.seg_stats);
+  hipLaunchKernelGGL(k_pcg_status, dim3(1), dim3(1024), 0, st, nseg, w.st, w.status);
+  FE_CHECK_LAUNCH();
+  FE_CHECK_HIP(hipMemcpyAsync(&pinned[0], w.status, sizeof(PcgStatus), hipMemcpyDeviceToHost, st));
+  if (flag) FE_CHECK_HIP(hipMemcpyAsync(&pinned[1], flag, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  FE_CHECK_HIP(hipStreamSynchronize(st));
+  s->iterations = pinned[0].max_iter;
+  s->reliable_updates = pinned[0].n_ru;
+  if (flag) *flag_out = *(const int32_t*)&pinned[1];
+  return FE_OK;
+}
+
+// The solve by a team of workgroups in one launch (fe_pcg_team.h): one segment on the padded pattern, of
+// at most kTeamMaxTiles tiles.  Beyond that the launches are long enough that their latency no longer
+// matters (64^3 cube: 2,152 tiles, 31 us of its 64 us iteration in the row product) and the matrix would
+// not stay on the chip.  Sets *ran when it was launched and *done when the solve has
+// ended; otherwise x holds a starting point and the caller runs the launched kernels.
+template <typename T, int D, int PC, int S>
+int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
+             bool* ran, bool* done) {
+  const fe_bsr* A64 = pb.A64;
+  const fe_bsr* Ait = pb.Ait;
+  hipStream_t st = h->stream;
+  const int rows = tile_rows_dof(D);
+  TeamArgs a{};
+  a.n_rows = (int32_t)A64->n_brows;
+  a.ntiles = (int32_t)ceil_div(A64->n_brows, rows);
+  a.pstride = (int32_t)pb.ntiles;
+  a.nnzb_it = Ait->nnzb;
+  a.nnzb = A64->nnzb;
+  a.bptr_it = Ait->bptr;
+  a.bcol_it = Ait->bcol;
+  a.bptr = A64->bptr;
+  a.bcol = A64->bcol;
+  a.vit = Ait->vals;
+  a.v64 = (const double*)A64->vals;
+  a.M = pb.M;
+  a.b = pb.b;
+  a.x = pb.x;
+  a.r = w.r;
+  a.u = w.u;
+  a.w = w.w;
+  a.p = w.p;
+  a.s = w.s;
+  a.r64 = w.r64;
+  a.st = w.st;
+  a.partials = w.partials;
+  a.flags = w.flags;
+  a.abort = (int32_t*)(w.flags + kTeamMaxTiles);
+  a.ut = w.ut;
+  a.pt = w.pt;
+  // LDS: u of the own rows, and of as many remote ones as fit beside the row bits and their ranks
+  const int64_t words = ceil_div(A64->n_brows, 32), fixed = kTeamLds - 6 * words - 16 - (int64_t)S * rows * D * sizeof(T);
+  a.lds_remote = (int32_t)std::min<int64_t>(65535, std::max<int64_t>(0, fixed / (int64_t)(D * sizeof(T) + 4)) / 4 * 4);
+  const int64_t lds = ((int64_t)S * rows + a.lds_remote) * D * sizeof(T) + 4 * (int64_t)a.lds_remote + 6 * words + 16;
+  a.chunk = chunk_of(o);
+  a.max_chunks = max_chunks_of(o);
+  const void* kernel = (const void*)k_pcg_team<T, D, PC, S>;
+  const int64_t grid = ceil_div(a.ntiles, S);
+  int per_cu = 0;
+  FE_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  FE_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock * S, (size_t)lds));
+  if (grid > (int64_t)per_cu * h->num_cus) return FE_OK;
+  FE_CHECK_HIP(hipMemsetAsync(w.flags, 0, (kTeamMaxTiles + 1) * sizeof(uint64_t), st));
+  void* args[] = {&a};
+  hipError_t e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)grid), dim3(kBlock * S), args, (unsigned)lds, st);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // this device or stream takes no cooperative launch
+    return FE_OK;
+  }
+  *ran = true;
+  int32_t aborted = 0;
+  int rc = finish_pcg(h, w, 1, s, a.abort, &aborted);
+  if (rc) return rc;
+  *done = aborted == 0;
+  return FE_OK;
+}
+
+template <typename T, int D, int PC>
+int try_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
+             bool* ran, bool* done) {
+  const int64_t tiles = ceil_div(pb.A64->n_brows, tile_rows_dof(D));
+  if (pb.nseg != 1 || pb.C || o->profile || !row_aligned(pb.Ait) || tiles > kTeamMaxTiles) return FE_OK;
+  // One workgroup per CU: the fewest threads per workgroup with which the chip holds the tiles, and up to
+  // two tiles in one workgroup, whose messages stay in its LDS (40 x 10 plate, two tiles: 1.2 ms against
+  // 2.3 ms by two workgroups).
+  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2>(h, pb, w, o, s, ran, done);
+  if (tiles <= 256) return run_team<T, D, PC, 1>(h, pb, w, o, s, ran, done);
+  // Four tiles per workgroup leave a thread 128 registers: enough in FP32 (40^3 cube, 539 tiles, block
+  // Jacobi: 61.9 -> 37.2 ms), not for FP64 vectors (47.7 ms launched, 50.5 ms in this form; 450^2
+  // magnetostatics 21.6 and 26.2 ms).
+  if constexpr (sizeof(T) == 4) return run_team<T, D, PC, 4>(h, pb, w, o, s, ran, done);
+  return FE_OK;
+}
+
 template <typename T, int D, int PC>
 int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s) {
   constexpr int G = lanes_for<D>();
@@ -754,13 +899,25 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
   const int nt = (int)pb.ntiles, nseg = pb.nseg;
   hipStream_t st = h->stream;
   const T* M = (const T*)pb.M;
+  const dim3 gt((unsigned)nt), gseg((unsigned)nseg);
+  auto launch_init = [&]() -> int {
+    hipLaunchKernelGGL((k_tile_norm<D>), gt, dim3(kBlock), 0, st, w.tiles, pb.b, w.partials);
+    hipLaunchKernelGGL(k_pcg_init, gseg, dim3(kRed), 0, st, w.seg_tiles, nt, w.partials, w.st, o->tol,
+                       o->max_iter, o->mixed, o->ru_delta);
+    FE_CHECK_LAUNCH();
+    return FE_OK;
+  };
+  {
+    int rc0 = launch_init();
+    if (rc0) return rc0;
+    bool ran = false, done = false;
+    rc0 = try_team<T, D, PC>(h, pb, w, o, s, &ran, &done);
+    if (rc0 || done) return rc0;
+    if (ran) rc0 = launch_init();  // the team gave up and left its state behind
+    if (rc0) return rc0;
+  }
   FE_CHECK_HIP(hipMemsetAsync(w.p, 0, n * sizeof(T), st));
   FE_CHECK_HIP(hipMemsetAsync(w.s, 0, n * sizeof(T), st));
-  const dim3 gt((unsigned)nt), gseg((unsigned)nseg);
-  hipLaunchKernelGGL((k_tile_norm<D>), gt, dim3(kBlock), 0, st, w.tiles, pb.b, w.partials);
-  hipLaunchKernelGGL(k_pcg_init, gseg, dim3(kRed), 0, st, w.seg_tiles, nt, w.partials, w.st, o->tol,
-                     o->max_iter, o->mixed, o->ru_delta);
-  FE_CHECK_LAUNCH();
   const int32_t* bptr = A64->bptr;
   const int32_t* bcol = A64->bcol;
   const double* v64 = (const double*)A64->vals;
@@ -801,7 +958,7 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
     if (rc0) return rc0;
   }
   FE_CHECK_LAUNCH();
-  const int chunk = o->check_every > 0 ? o->check_every : 16;
+  const int chunk = chunk_of(o);
   PcgStatus* pinned = (PcgStatus*)h->pinned;
   hipEvent_t ev[2];
   FE_CHECK_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
@@ -874,7 +1031,7 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
   // trend of the last two polls predicts that the chunk already queued ends the solve: then the host
   // waits for it before queueing another (a chunk queued after convergence finds every segment done
   // and returns at once, but its launches still cost device time).
-  const int64_t max_chunks = 4 * ((int64_t)o->max_iter / chunk + 2) + 8;
+  const int64_t max_chunks = max_chunks_of(o);
   PcgStatus last{};
   int finished = 0;
   int64_t queued = 0, polled = 0;
@@ -934,16 +1091,7 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
     (void)hipEventDestroy(p0);
     (void)hipEventDestroy(p1);
   }
-  hipLaunchKernelGGL(k_pcg_export, dim3((unsigned)ceil_div(nseg, 256)), dim3(256), 0, st, nseg, w.st,
-                     w.seg_stats);
-  hipLaunchKernelGGL(k_pcg_status, dim3(1), dim3(1024), 0, st, nseg, w.st, w.status);
-  FE_CHECK_LAUNCH();
-  FE_CHECK_HIP(hipMemcpyAsync(&pinned[0], w.status, sizeof(PcgStatus), hipMemcpyDeviceToHost, st));
-  FE_CHECK_HIP(hipStreamSynchronize(st));
-  last = pinned[0];
-  s->iterations = last.max_iter;
-  s->reliable_updates = last.n_ru;
-  return FE_OK;
+  return finish_pcg(h, w, nseg, s, nullptr, nullptr);
 }
 
 template <typename T, int D>

@@ -17,10 +17,58 @@ __device__ __host__ inline int64_t vix(int64_t q, int k, int64_t nnzb) {
 // --------------------------------------------------------------------------------------------------
 // reductions
 // --------------------------------------------------------------------------------------------------
+// Sum over the wavefront, in every lane: the butterfly over lane distances 32, 16, 8, 4, 2, 1.  The exchanges
+// are register moves (swaps of half wavefronts and of rows, then lane permutations inside a row of 16):
+// six dependent LDS permutes took 0.35 us, on the critical path of every reduction.  Once two
+// distances have been added, all lanes they connect hold the same bits, so a rotation by 8 and by
+// 4 lanes within the row of 16 meets a lane with the value the butterfly's partner holds.
+template <int CTRL>
+__device__ inline double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int CTRL>
+__device__ inline float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  long long b = __double_as_longlong(v);
+  u2 l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  u2 h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+  b = __double_as_longlong(v);
+  l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+  h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+  v += dpp_move<0x128>(v);  // row_ror:8
+  v += dpp_move<0x124>(v);  // row_ror:4
+  v += dpp_move<0x4e>(v);   // quad_perm [2,3,0,1]
+  return v + dpp_move<0xb1>(v);  // quad_perm [1,0,3,2]
+}
+
+// Sum over the aligned group of G lanes (2, 4, 8 or 16) that share a row, in every lane, over the lane
+// distances 1, 2, 4, 8: from 4 on a mirror image meets a lane of the other half, and all of a half's lanes
+// hold its sum.
+template <int G, typename T>
+__device__ inline T group_sum(T v) {
+  static_assert(G == 2 || G == 4 || G == 8 || G == 16, "lanes of one row of 16");
+  v += dpp_move<0xb1>(v);
+  if constexpr (G >= 4) v += dpp_move<0x4e>(v);
+  if constexpr (G >= 8) v += dpp_move<0x141>(v);   // row_half_mirror
+  if constexpr (G >= 16) v += dpp_move<0x140>(v);  // row_mirror
   return v;
+}
+
+// Lane J's value of the group of G lanes, for the lanes 0..3 of the group (J < 4).
+template <int G, int J, typename T>
+__device__ inline T group_lane(T v) {
+  static_assert(J < G && J < 4, "a lane of the group's first four");
+  constexpr int kCtrl = G == 2 ? (J | J << 2 | (2 + J) << 4 | (2 + J) << 6) : (J | J << 2 | J << 4 | J << 6);
+  return dpp_move<kCtrl>(v);
 }
 
 // Sum NV values over the workgroup; result valid in thread 0.
@@ -65,9 +113,7 @@ __device__ inline void bsr_row(const int32_t* __restrict__ bptr, const int32_t* 
       for (int dj = 0; dj < D; ++dj) acc[di] += vals[vix<D, LAYOUT>(q, di * D + dj, nnzb)] * xj[dj];
   }
 #pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1)
-#pragma unroll
-    for (int d = 0; d < D; ++d) acc[d] += __shfl_xor(acc[d], off, G);
+  for (int d = 0; d < D; ++d) acc[d] = group_sum<G>(acc[d]);
 }
 
 // 16-byte vectors: W = 16 / sizeof(T) consecutive entries of one value plane, and their columns.
@@ -119,9 +165,7 @@ __device__ inline void bsr_row_vec_range(const int32_t* __restrict__ bcol, const
     }
   }
 #pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1)
-#pragma unroll
-    for (int d = 0; d < D; ++d) acc[d] += __shfl_xor(acc[d], off, G);
+  for (int d = 0; d < D; ++d) acc[d] = group_sum<G>(acc[d]);
 }
 
 template <typename T, int D, int G>

@@ -151,6 +151,9 @@ SIGNATURES = {
     'fe_pcg_coarse_workspace': (_int, [_vp, _P(FeBsr), _P(FeCoarse), _P(FePcgOpts), _P(_i64)]),
     'fe_pcg_coarse': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _P(FeCoarse), _vp, _vp, _vp, _vp,
                              _vp, _i64, _P(FePcgOpts), _P(FePcgStats)]),
+    'fe_pcg_coarse_takes_ordered': (_int, [_P(FeBsr), _P(FeCoarse), _P(FePcgOpts), _P(_int)]),
+    'fe_pcg_coarse_ordered': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _P(FeCoarse), _vp, _vp, _vp, _vp,
+                                     _i64, _P(FePcgOpts), _P(FePcgStats)]),
     'fe_pcg_batched_coarse_workspace': (_int, [_vp, _P(FeBsr), _i32, _vp, _P(FeCoarse), _P(FePcgOpts),
                                                _P(_i64)]),
     'fe_pcg_batched_coarse': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _i32, _vp, _P(FeCoarse), _vp, _vp,

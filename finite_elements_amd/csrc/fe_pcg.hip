@@ -715,6 +715,8 @@ struct Work {
   uint64_t* flags;  // the team's arrival flags, then its abort word
   uint64_t* ut;     // its messages: u, and the partial dots
   uint64_t* pt;
+  char* ring;       // its moments, and B = T A_c^-1 T^T (two-level)
+  void* binv;
   fe_pcg_seg_stats* seg_stats;
   void* r;
   void* u;
@@ -732,6 +734,11 @@ int64_t count_tiles(int nseg, const int32_t* seg_nodes, int rows) {
   int64_t t = 0;
   for (int g = 0; g < nseg; ++g) t += ceil_div((int64_t)seg_nodes[g + 1] - seg_nodes[g], rows);
   return t == 0 ? 0 : (t + 7) / 8 * 8;  // padded with empty tiles to a multiple of the 8 XCDs
+}
+
+// Bytes of a region: the parts t + g of nwg workgroups (n_agg: their aggregates, or a bound on them).
+inline int64_t team_region(int64_t nwg, int64_t ntiles, int64_t n_agg, int NC, int elem) {
+  return team_part(nwg + 1, ntiles + n_agg, NC, elem) + 256;
 }
 
 Work layout_work(char* base, int64_t nb, int dof, int elem, int nseg, int64_t ntiles,
@@ -753,6 +760,9 @@ Work layout_work(char* base, int64_t nb, int dof, int elem, int nseg, int64_t nt
   w.flags = (uint64_t*)take((kTeamMaxTiles + 1) * (int64_t)sizeof(uint64_t));
   w.ut = (uint64_t*)take(team ? n * 2 * (int64_t)sizeof(uint64_t) : 0);
   w.pt = (uint64_t*)take(team ? 12 * kTeamCopies * std::max<int64_t>(1, ntiles) * (int64_t)sizeof(uint64_t) : 0);
+  const bool team_co = team && n_coarse > 0 && n_coarse <= kTeamMaxCoarse;
+  w.ring = (char*)take(team_co ? kTeamRing * team_region(std::min<int64_t>(ntiles, 256), ntiles, n_coarse, 6, 8) : 0);
+  w.binv = take(team_co ? n_coarse * fe_coarse_ld(n_coarse) * (int64_t)sizeof(double) : 0);
   w.seg_stats = (fe_pcg_seg_stats*)take(nseg * (int64_t)sizeof(fe_pcg_seg_stats));
   w.r = take(n * elem);
   w.u = take(n * elem);
@@ -776,7 +786,11 @@ struct Problem {
   int64_t ntiles;
   const fe_coarse* C;  // two-level: coarse space and the inverse coarse operator (iteration precision)
   const void* Ainv;
+  const void* Ainv64;  // ordered: Ait's rows and columns are the nodes as C->agg_nodes lists them (the team's
+  bool ordered;        // form; the launched kernels do not take it), with the FP64 inverse
 };
+
+constexpr int kErrTeamLeft = 1000;  // internal: an ordered solve that the team did not finish
 
 inline int chunk_of(const fe_pcg_opts* o) { return o->check_every > 0 ? o->check_every : 16; }
 inline int64_t max_chunks_of(const fe_pcg_opts* o) {
@@ -806,7 +820,7 @@ int finish_pcg(fe_handle* h, const Work& w, int nseg, fe_pcg_stats* s, const int
 // matters (64^3 cube: 2,152 tiles, 31 us of its 64 us iteration in the row product) and the matrix would
 // not stay on the chip.  Sets *ran when it was launched and *done when the solve has
 // ended; otherwise x holds a starting point and the caller runs the launched kernels.
-template <typename T, int D, int PC, int S>
+template <typename T, int D, int PC, int S, bool CO>
 int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
              bool* ran, bool* done) {
   const fe_bsr* A64 = pb.A64;
@@ -840,19 +854,38 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   a.abort = (int32_t*)(w.flags + kTeamMaxTiles);
   a.ut = w.ut;
   a.pt = w.pt;
-  // LDS: u of the own rows, and of as many remote ones as fit beside the row bits and their ranks
-  const int64_t words = ceil_div(A64->n_brows, 32), fixed = kTeamLds - 6 * words - 16 - (int64_t)S * rows * D * sizeof(T);
-  a.lds_remote = (int32_t)std::min<int64_t>(65535, std::max<int64_t>(0, fixed / (int64_t)(D * sizeof(T) + 4)) / 4 * 4);
-  const int64_t lds = ((int64_t)S * rows + a.lds_remote) * D * sizeof(T) + 4 * (int64_t)a.lds_remote + 6 * words + 16;
+  // LDS: u of the own rows, and of as many remote ones as fit beside the rest
+  constexpr int NC = D == 1 ? 1 : D == 2 ? 3 : 6;
+  const int64_t rest = team_lds(A64->n_brows, S * rows, CO ? pb.C->n_agg : 0, D, NC, (int)sizeof(T)).total;
+  const int64_t room = kTeamLds - rest - (int64_t)S * rows * D * sizeof(T);
+  if (room < 0) return FE_OK;
+  a.lds_remote = (int32_t)std::min<int64_t>(65532, room / (int64_t)(D * sizeof(T) + 4) / 4 * 4);
+  const int64_t lds = ((int64_t)S * rows + a.lds_remote) * D * sizeof(T) + 4 * (int64_t)a.lds_remote + rest;
+  if constexpr (CO) {
+    const fe_coarse* C = pb.C;
+    a.order = C->agg_nodes;
+    a.agg_ptr = C->agg_ptr;
+    a.node_agg = C->node_agg;
+    a.xhat = sizeof(T) == 4 ? (const void*)C->xhat32 : (const void*)C->xhat;
+    a.fixed_bits = C->fixed_bits;
+    a.n_agg = (int32_t)C->n_agg;
+    a.ldb = fe_coarse_ld(C->n_agg * NC);
+    a.B = w.binv;
+    a.ring = w.ring;
+    a.region = team_region(ceil_div(a.ntiles, S), a.ntiles, pb.C->n_agg, NC, (int)sizeof(T));
+  }
   a.chunk = chunk_of(o);
   a.max_chunks = max_chunks_of(o);
-  const void* kernel = (const void*)k_pcg_team<T, D, PC, S>;
+  const void* kernel = (const void*)k_pcg_team<T, D, PC, S, CO>;
   const int64_t grid = ceil_div(a.ntiles, S);
   int per_cu = 0;
   FE_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   FE_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock * S, (size_t)lds));
   if (grid > (int64_t)per_cu * h->num_cus) return FE_OK;
   FE_CHECK_HIP(hipMemsetAsync(w.flags, 0, (kTeamMaxTiles + 1) * sizeof(uint64_t), st));
+  if constexpr (CO)
+    hipLaunchKernelGGL((k_team_binv<T, NC>), dim3((unsigned)ceil_div(pb.C->n_agg * pb.C->n_agg, 64)), dim3(64), 0, st,
+                       (int32_t)pb.C->n_agg, (const double*)pb.Ainv64, a.ldb, pb.C->T, (T*)w.binv);
   void* args[] = {&a};
   hipError_t e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)grid), dim3(kBlock * S), args, (unsigned)lds, st);
   if (e != hipSuccess) {
@@ -867,20 +900,30 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   return FE_OK;
 }
 
-template <typename T, int D, int PC>
+// Whether a system of this size, precision and coarse space (n_coarse 0: none) is the team's.
+inline bool team_takes(int64_t n_rows, int dof, int elem, int64_t n_coarse) {
+  const int64_t tiles = ceil_div(n_rows, tile_rows_dof(dof));
+  // Four tiles per workgroup (above 512) leave a thread 128 registers: enough in FP32 (40^3 cube, 539
+  // tiles, block Jacobi: 61.9 -> 37.2 ms), not for FP64 vectors (47.7 ms launched, 50.5 ms in this
+  // form; 450^2 magnetostatics 21.6 and 26.2 ms) unless the launched form has the coarse correction's three
+  // kernels more and the blocks are small (450^2 magnetostatics, two-level FP64: 8.4 -> 6.6 ms; 40^3
+  // cube 11.6 ms either way).
+  const bool four = elem == 4 || (n_coarse > 0 && dof <= 2);
+  return tiles <= (four ? kTeamMaxTiles : kTeamMaxTiles / 2) && n_coarse <= kTeamMaxCoarse;
+}
+
+template <typename T, int D, int PC, bool CO>
 int try_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
              bool* ran, bool* done) {
   const int64_t tiles = ceil_div(pb.A64->n_brows, tile_rows_dof(D));
-  if (pb.nseg != 1 || pb.C || o->profile || !row_aligned(pb.Ait) || tiles > kTeamMaxTiles) return FE_OK;
+  const int64_t nct = CO ? pb.C->n_agg * pb.C->nc : 0;
+  if (!team_takes(pb.A64->n_brows, D, (int)sizeof(T), nct)) return FE_OK;
   // One workgroup per CU: the fewest threads per workgroup with which the chip holds the tiles, and up to
   // two tiles in one workgroup, whose messages stay in its LDS (40 x 10 plate, two tiles: 1.2 ms against
   // 2.3 ms by two workgroups).
-  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2>(h, pb, w, o, s, ran, done);
-  if (tiles <= 256) return run_team<T, D, PC, 1>(h, pb, w, o, s, ran, done);
-  // Four tiles per workgroup leave a thread 128 registers: enough in FP32 (40^3 cube, 539 tiles, block
-  // Jacobi: 61.9 -> 37.2 ms), not for FP64 vectors (47.7 ms launched, 50.5 ms in this form; 450^2
-  // magnetostatics 21.6 and 26.2 ms).
-  if constexpr (sizeof(T) == 4) return run_team<T, D, PC, 4>(h, pb, w, o, s, ran, done);
+  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2, CO>(h, pb, w, o, s, ran, done);
+  if (tiles <= 256) return run_team<T, D, PC, 1, CO>(h, pb, w, o, s, ran, done);
+  if constexpr (sizeof(T) == 4 || (CO && D <= 2)) return run_team<T, D, PC, 4, CO>(h, pb, w, o, s, ran, done);
   return FE_OK;
 }
 
@@ -911,7 +954,11 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
     int rc0 = launch_init();
     if (rc0) return rc0;
     bool ran = false, done = false;
-    rc0 = try_team<T, D, PC>(h, pb, w, o, s, &ran, &done);
+    if (pb.ordered) {
+      if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, &ran, &done);
+      return rc0 ? rc0 : done ? FE_OK : kErrTeamLeft;
+    }
+    if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, &ran, &done);
     if (rc0 || done) return rc0;
     if (ran) rc0 = launch_init();  // the team gave up and left its state behind
     if (rc0) return rc0;
@@ -1151,7 +1198,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
                int nseg, const int32_t* seg_nodes, const double* b, double* x, void* work,
                int64_t work_bytes, const fe_pcg_opts* o, fe_pcg_stats* s, fe_pcg_seg_stats* seg_out,
                const char* who, const fe_coarse* C = nullptr, const void* Ainv64 = nullptr,
-               const void* Ainv32 = nullptr) {
+               const void* Ainv32 = nullptr, bool ordered = false) {
   const int elem = (int)sizeof(double);  // FP64-sized vectors: the FP64 fallback reuses them
   const int rows = tile_rows_dof(A64->dof);
   const int64_t ntiles = count_tiles(nseg, seg_nodes, rows);
@@ -1178,11 +1225,18 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
                               hipMemcpyHostToDevice, h->stream));
   // the block-diagonal coarse space applies its FP64 blocks at every precision
   Problem pb{A64, A32 ? A32 : A64, o->mixed ? M32 : M64, b, x, nseg, ntiles, C,
-             (o->mixed && !(C && C->n_seg)) ? Ainv32 : Ainv64};
+             (o->mixed && !(C && C->n_seg)) ? Ainv32 : Ainv64, Ainv64, ordered};
   *s = fe_pcg_stats{};
   int rc = ntiles == 0 ? FE_OK
            : o->mixed  ? dispatch_dof<float>(h, pb, w, o, s)
                        : dispatch_dof<double>(h, pb, w, o, s);
+  fe_pcg_opts o_plain = *o;
+  if (rc == kErrTeamLeft) {
+    // the launched kernels finish an ordered solve in FP64, on A64 itself
+    o_plain.mixed = 0;
+    Problem plain{A64, A64, M64, b, x, nseg, ntiles, C, Ainv64, Ainv64, false};
+    rc = dispatch_dof<double>(h, plain, w, &o_plain, s);
+  }
   if (rc) {
     (void)hipStreamSynchronize(h->stream);  // the host tile arrays must outlive their copies
     return rc;
@@ -1200,7 +1254,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
   // segments that already converged stop at the first true-residual check
   int failed = 0;
   for (const auto& q : seg) failed += q.status != FE_OK;
-  if (o->mixed && M64 && failed && ntiles > 0 && (!C || Ainv64)) {
+  if (o_plain.mixed && M64 && failed && ntiles > 0 && (!C || Ainv64)) {
     // a segment that ended worse than the zero vector restarts from zero
     const int D = A64->dof;
     for (int g = 0; g < nseg; ++g)
@@ -1211,7 +1265,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
     fe_pcg_opts o64 = *o;
     o64.mixed = 0;
     o64.profile = 0;
-    Problem pb64{A64, A64, M64, b, x, nseg, ntiles, C, Ainv64};
+    Problem pb64{A64, A64, M64, b, x, nseg, ntiles, C, Ainv64, Ainv64, false};
     fe_pcg_stats s64{};
     rc = dispatch_dof<double>(h, pb64, w, &o64, &s64);
     if (rc) return rc;
@@ -1332,6 +1386,35 @@ extern "C" int fe_pcg_coarse(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32,
   const int32_t seg[2] = {0, (int32_t)A64->n_brows};
   return pcg_common(h, A64, A32, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr,
                     "fe_pcg_coarse", C, Ainv64, Ainv32);
+}
+
+extern "C" int fe_pcg_coarse_takes_ordered(const fe_bsr* A, const fe_coarse* C, const fe_pcg_opts* o, int* yes) {
+  FE_REQUIRE(A && C && o && yes, "fe_pcg_coarse_takes_ordered: null argument");
+  FE_REQUIRE(A->dof >= 1 && A->dof <= 3, "fe_pcg_coarse_takes_ordered: dof must be 1..3");
+  *yes = o->precond == FE_PC_BLOCK_JACOBI && !o->profile && C->n_seg == 0 && C->fixed_bits && C->T &&
+         (o->mixed ? C->xhat32 != nullptr : C->xhat != nullptr) && A->n_brows > 0 &&
+         team_takes(A->n_brows, A->dof, o->mixed ? 4 : 8, C->n_agg * C->nc);
+  return FE_OK;
+}
+
+extern "C" int fe_pcg_coarse_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
+                                     const void* M32, const fe_coarse* C, const void* Ainv64, const double* b,
+                                     double* x, void* work, int64_t work_bytes, const fe_pcg_opts* o,
+                                     fe_pcg_stats* s) {
+  FE_ENTER(h);
+  FE_REQUIRE(b && x && work && o && s && C && A64 && Aord && M64 && Ainv64, "fe_pcg_coarse_ordered: null argument");
+  int rc = check_pcg_args(A64, Aord, M64, M32, o, "fe_pcg_coarse_ordered");
+  if (rc) return rc;
+  int yes = 0;
+  rc = fe_pcg_coarse_takes_ordered(A64, C, o, &yes);
+  if (rc) return rc;
+  FE_REQUIRE(yes, "fe_pcg_coarse_ordered: not a system for the ordered form (fe_pcg_coarse_takes_ordered)");
+  FE_REQUIRE(Aord->row_align == 4, "fe_pcg_coarse_ordered: the iteration matrix must be on a padded pattern");
+  FE_REQUIRE(C->dof == A64->dof && C->n_nodes == A64->n_brows, "fe_pcg_coarse_ordered: coarse space and A disagree");
+  *s = fe_pcg_stats{};
+  const int32_t seg[2] = {0, (int32_t)A64->n_brows};
+  return pcg_common(h, A64, Aord, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr,
+                    "fe_pcg_coarse_ordered", C, Ainv64, nullptr, true);
 }
 
 extern "C" int fe_pcg_batched_coarse_workspace(fe_handle* h, const fe_bsr* A, int32_t n_seg,

@@ -16,11 +16,27 @@
 // flag).  The reliable updates (a few per solve) use flags.  The matrix, or where it is too wide its
 // columns, stays in registers for the whole solve; vectors are in registers between updates.
 // Per iteration, launched kernels and this: 40 x 10 plate FP64 (one workgroup) 11.2 -> 3.2 us, 13^3 cube
-// FP64 (22 workgroups) 17 -> 6.2 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.2 us.
+// FP64 (22 workgroups) 17 -> 6.2 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.2 us; two-level mixed 27^3 cube
+// (172) 40 -> 14 us, 450^2 magnetostatics (199) 33 -> 13 us.
+//
+// Two-level preconditioner (CO): the node rows are numbered aggregate by aggregate (order), so that a
+// workgroup's rows touch few aggregates.  The correction P A_c^-1 P^T r is carried by the recurrence of r:
+// with z, zeta and y the corrections of r, s and w, s = w + beta s gives zeta = y + beta zeta and
+// r -= alpha s gives z -= alpha zeta, so an iteration needs P^T w only.  Every tile sums the rigid-body
+// moments of its rows of w by aggregate and hands them over with its partial dots; every workgroup adds
+// all of them up and applies the rows of B = T A_c^-1 T^T that its own aggregates need.  The correction costs no
+// further meeting (launched: three kernels per iteration).  The reliable updates form z, zeta and y anew.
+// All workgroups read all moments, a few KB that message words and agent-scope loads would fetch from
+// memory once per workgroup (450^2 magnetostatics, 199 workgroups: 16 us per iteration).  So here the
+// moments and dots are stored first, by agent-scope stores, then a flag, and read by plain loads, which
+// the workgroups of an XCD share through its L2.  That is sound because a meeting's region of memory has not
+// been read since the last invalidation: the regions are a ring of kTeamRing, and every wavefront
+// invalidates (agent-scope acquire fence) before it reads the ring's first region; a workgroup's part of a
+// region begins on a cache line of its own.
 //
 // The arithmetic -- tiles, row products, partial sums and their order, the scalars, reliable updates at
-// chunk ends -- is that of the launched kernels (fe_pcg.hip), so a system solved here has the bits of
-// the same system solved as a segment of a batch.
+// chunk ends -- is that of the launched kernels (fe_pcg.hip), so a system solved here without a
+// coarse correction has the bits of the same system solved as a segment of a batch.
 //
 // The launch is cooperative (all workgroups resident, cooperative launches never side by side).  Every
 // wait is bounded: a workgroup that has polled kTeamSpins times raises `abort` and leaves, the others
@@ -34,6 +50,8 @@ namespace {
 constexpr int kTeamMaxTiles = 1024;
 constexpr int kTeamSpins = 1 << 21;  // polls of about a microsecond
 constexpr int kTeamCopies = 8;  // of the partial dots: a workgroup reads copy blockIdx.x % 8
+constexpr int kTeamMaxCoarse = 1536;  // coarse DOF: every workgroup holds all their moments in LDS
+constexpr int kTeamRing = 64;   // regions of the moments' ring
 constexpr int kTeamLds = 144 * 1024;  // dynamic LDS of a workgroup, of the CU's 160 KB
 
 struct TeamArgs {
@@ -56,7 +74,78 @@ struct TeamArgs {
   int32_t lds_remote;  // remote node rows whose u fits in LDS
   int32_t chunk;
   int64_t max_chunks;
+  // two-level: node rows by aggregate (row i of the iteration matrix is node order[i]), the aggregates'
+  // row ranges, their nodes' x^ and constraint bits, B (iteration precision, leading dimension ldb) and
+  // the ring of kTeamRing regions of region bytes
+  const int32_t *order, *agg_ptr, *node_agg;
+  const void* xhat;
+  const uint8_t* fixed_bits;
+  const void* B;
+  int64_t ldb;
+  int32_t n_agg;
+  char* ring;
+  int64_t region;
 };
+
+// B = T A_c^-1 T^T by blocks (I, J) of coarse DOF: the correction in rigid-body moments and motions.
+template <typename T, int NC>
+__global__ __launch_bounds__(64) void k_team_binv(int32_t n_agg, const double* __restrict__ Ainv, int64_t ld,
+                                                  const double* __restrict__ Tm, T* __restrict__ B) {
+  const int64_t t = blockIdx.x * (int64_t)64 + threadIdx.x;
+  if (t >= (int64_t)n_agg * n_agg) return;
+  const int64_t I = t / n_agg, J = t % n_agg;
+  double a[NC][NC], q[NC][NC];
+#pragma unroll
+  for (int x = 0; x < NC; ++x)
+#pragma unroll
+    for (int y = 0; y < NC; ++y) a[x][y] = Ainv[(I * NC + x) * ld + J * NC + y];
+#pragma unroll
+  for (int x = 0; x < NC; ++x)
+#pragma unroll
+    for (int y = 0; y < NC; ++y) {
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) v += a[x][k] * Tm[(J * NC + y) * NC + k];
+      q[x][y] = v;
+    }
+#pragma unroll
+  for (int x = 0; x < NC; ++x)
+#pragma unroll
+    for (int y = 0; y < NC; ++y) {
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) v += Tm[(I * NC + x) * NC + k] * q[k][y];
+      B[(I * NC + x) * ld + J * NC + y] = (T)v;
+    }
+}
+
+// A region of the ring: workgroup b's three partial dots, then the moments of its parts, the first of them
+// part q0; its place leaves whole cache lines to the workgroups before it.
+inline __host__ __device__ int64_t team_part(int64_t b, int64_t q0, int NC, int elem) {
+  return 128 * (2 * b + q0 * NC * elem / 128);
+}
+constexpr int kTeamDots = 32;  // bytes of the dots ahead of the moments
+
+// Dynamic LDS of a workgroup: the parts beside u's, which take the rest.
+struct TeamLds {
+  int64_t bits, wl, xl, fb, ap, zs, total;  // byte offsets from the end of rlist, and their sum
+};
+inline __host__ __device__ TeamLds team_lds(int64_t n_rows, int64_t wg_rows, int64_t n_agg, int D, int NC, int elem) {
+  TeamLds l{};
+  auto take = [&](int64_t& at, int64_t bytes) {
+    at = l.total;
+    l.total += (bytes + 15) / 16 * 16;
+  };
+  take(l.bits, (n_rows + 31) / 32 * 6);
+  if (n_agg > 0) {
+    take(l.wl, wg_rows * D * elem);
+    take(l.xl, D == 1 ? 0 : wg_rows * 3 * elem);
+    take(l.fb, wg_rows);
+    take(l.ap, (n_agg + 1) * 4);
+    take(l.zs, n_agg * NC * 8);
+  }
+  return l;
+}
 
 template <typename V>
 __device__ inline V ld_team(const V* p) {
@@ -124,7 +213,7 @@ constexpr bool team_resident() {
   return regs <= (S == 1 ? 168 : S == 2 ? 80 : 40);
 }
 
-template <typename T, int D, int PC, int S>
+template <typename T, int D, int PC, int S, bool CO>
 __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   using V = typename Vec16<T>::V;
   using I = typename Vec16<T>::I;
@@ -134,6 +223,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   constexpr int kRows = kBlock / GV;              // rows per pass of the iteration's row product
   constexpr int kPasses = R / kRows;
   constexpr int NM = PC == FE_PC_JACOBI ? 1 : D;
+  constexpr int NC = D == 1 ? 1 : D == 2 ? 3 : 6;  // rigid-body modes of an aggregate
   constexpr int NT = kBlock * S;
   constexpr int TW = team_words<T>();
   constexpr bool kRes = team_resident<T, D, S>();
@@ -145,14 +235,24 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   __shared__ double s_sum[5][kWaves];
   __shared__ int s_fail, s_lo, s_hi;
   __shared__ int s_scan[NT];
+  __shared__ int s_q0[CO ? 256 : 1];
   // u by local row: this workgroup's S R rows, then the rows of others that its blocks touch (rlist,
   // ascending); a bit per row of the system for the latter, and the number of bits before each word
   extern __shared__ __align__(16) char s_dyn[];
   T* ul = (T*)s_dyn;
   int32_t* rlist = (int32_t*)(s_dyn + (size_t)(S * R + a.lds_remote) * D * sizeof(T));
-  uint32_t* bits = (uint32_t*)(rlist + a.lds_remote);
+  char* s_rest = (char*)(rlist + a.lds_remote);
+  const TeamLds at_lds = team_lds(a.n_rows, S * R, CO ? a.n_agg : 0, D, NC, (int)sizeof(T));
+  uint32_t* bits = (uint32_t*)(s_rest + at_lds.bits);
   const int nwords = (a.n_rows + 31) / 32;
   uint16_t* rank = (uint16_t*)(bits + nwords);
+  // two-level: a vector and the nodes' x^ and constraint bits by own row, the aggregates' row ranges and the
+  // coarse vectors
+  T* wl_ = (T*)(s_rest + at_lds.wl);
+  T* xl = (T*)(s_rest + at_lds.xl);
+  uint8_t* fb = (uint8_t*)(s_rest + at_lds.fb);
+  int32_t* aggp = (int32_t*)(s_rest + at_lds.ap);
+  double* cm = (double*)(s_rest + at_lds.zs);
 
   const int sub = threadIdx.x / kBlock, tid = threadIdx.x % kBlock;
   const int wl = threadIdx.x & 63, wid = tid >> 6;
@@ -215,7 +315,14 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     __syncthreads();
   }
   const int nr = s_scan[NT - 1];  // remote rows
-  const bool fits = nr <= a.lds_remote;
+  // two-level: behind the remote rows' u, the coarse vectors of the workgroup's aggregates
+  int g0 = 0, ng = 0;
+  if constexpr (CO) {
+    g0 = a.node_agg[a.order[wr0]];
+    ng = (wr1 > wr0 ? a.node_agg[a.order[wr1 - 1]] : g0) - g0 + 1;
+  }
+  const int co_rows = (3 * ng * NC * 8 + 16 + D * (int)sizeof(T) - 1) / (D * (int)sizeof(T));  // in rows of u
+  const bool fits = nr + (CO ? co_rows : 0) <= a.lds_remote;
   int at = s_scan[threadIdx.x] - count;
   for (int k = w0; k < w1; ++k) {
     rank[k] = (uint16_t)at;
@@ -237,7 +344,8 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
     for (int j = 0; j < NM; ++j) mk[ps][j] = T(0);
     if (i < row1 && lane < D) {
-      const T* m = PC == FE_PC_JACOBI ? M + (int64_t)i * D + lane : M + (int64_t)i * D * D + lane * D;
+      const int64_t node = CO ? a.order[i] : i;
+      const T* m = PC == FE_PC_JACOBI ? M + node * D + lane : M + node * D * D + lane * D;
 #pragma unroll
       for (int j = 0; j < NM; ++j) mk[ps][j] = m[j];
     }
@@ -434,13 +542,18 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     k = (int64_t)i * D + lane;
     return lane < D && i < row1;
   };
+  // the DOF's place in the caller's vectors (x, b)
+  auto caller = [&](int ps, int64_t k) -> int64_t {
+    if constexpr (!CO) return k;
+    return (int64_t)a.order[team_here(my_row) + ps * kRows] * D + lane;
+  };
 #pragma unroll
   for (int ps = 0; ps < kPasses; ++ps) {
     int64_t k;
     pk[ps] = sk[ps] = rk[ps] = wk[ps] = uk[ps] = T(0);
     xk[ps] = 0.0;
     if (own(ps, k)) {
-      xk[ps] = a.x[k];
+      xk[ps] = a.x[caller(ps, k)];
       // words of an earlier solve could carry this one's numbers: cleared ahead of the first meeting
 #pragma unroll
       for (int h = 0; h < TW; ++h) st_team(a.ut + k * TW + h, (uint64_t)0);
@@ -463,6 +576,201 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     }
   };
 
+  // ---- coarse correction (CO) -----------------------------------------------------------------------
+  const int n_c = CO ? a.n_agg * NC : 0;
+  double* zc = (double*)(s_dyn + (((size_t)(S * R + nr) * D * sizeof(T) + 15) & ~(size_t)15));
+  double *ze = zc + ng * NC, *yc = ze + ng * NC;
+  int tg0 = 0, tg1 = -1;
+  if constexpr (CO) {
+    // the tile's parts: its aggregates, from that of the row before it (an empty part where the tile starts
+    // one), so that the parts of all tiles are numbered tile + aggregate without a gap
+    if (tile < a.ntiles) {
+      tg0 = row0 > 0 ? a.node_agg[a.order[row0 - 1]] : 0;
+      tg1 = a.node_agg[a.order[row1 - 1]];
+    }
+    for (int32_t i = wr0 + (int)threadIdx.x; i < wr1; i += NT) {
+      const int64_t node = a.order[i];
+      fb[i - wr0] = a.fixed_bits[node];
+      if constexpr (D > 1)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) xl[(i - wr0) * 3 + c] = ((const T*)a.xhat)[node * 3 + c];
+    }
+  }
+  int32_t la[kPasses];  // first of the node's aggregate's entries in zc, or -1 where the DOF is constrained
+#pragma unroll
+  for (int ps = 0; ps < kPasses; ++ps) {
+    la[ps] = -1;
+    if constexpr (CO) {
+      const int32_t i = row0 + ps * kRows + tid / GV;
+      if (lane < D && i < row1) {
+        const int32_t node = a.order[i];
+        if (!((a.fixed_bits[node] >> lane) & 1)) la[ps] = (a.node_agg[node] - g0) * NC;
+      }
+    }
+  }
+  const int nwg = (int)gridDim.x;
+  if constexpr (CO)
+    for (int g = threadIdx.x; g < nwg; g += NT) {
+      const int32_t row = g * S * R;
+      s_q0[g] = g * S + (row > 0 ? a.node_agg[a.order[row - 1]] : 0);
+    }
+  if constexpr (CO)
+    for (int g = threadIdx.x; g <= a.n_agg; g += NT) aggp[g] = a.agg_ptr[g];
+  constexpr int kParts = 2;
+  int turn = 0;  // region of the ring
+  // the rows of B that this workgroup applies, in LDS behind the remote rows where they fit
+  const T* Brows = (const T*)a.B + (int64_t)g0 * NC * a.ldb;
+  int64_t ldb = a.ldb;
+  if constexpr (CO) {
+    if (fits && (int64_t)ng * NC * n_c <= (int64_t)(a.lds_remote - nr - co_rows) * D) {
+      T* Bl = (T*)(yc + ng * NC);
+      for (int q = (int)threadIdx.x / 64; q < ng * NC; q += NT / 64)
+        for (int c = wl; c < n_c; c += 64) Bl[q * n_c + c] = Brows[q * ldb + c];
+      Brows = Bl;
+      ldb = n_c;
+    }
+  }
+  auto coarse_rows = [&](const T* v) {
+#pragma unroll
+    for (int ps = 0; ps < kPasses; ++ps) {
+      const int32_t i = team_here(my_row) + ps * kRows;
+      if (lane < D && i < row1) wl_[(i - wr0) * D + lane] = v[ps];
+    }
+  };
+  // A meeting of all for the moments of the rows in wl_ and, if v3, the dots' wavefront sums in s_red (both
+  // behind a barrier): c in cm, the dots' sums over the workgroups' wavefronts in s_sum.
+  auto coarse_meet = [&](bool dots) {
+    char* region = a.ring + turn * a.region;
+    if (++turn == kTeamRing) turn = 0;
+    const int q0 = s_q0[blockIdx.x];
+    char* mine = region + team_part(blockIdx.x, q0, NC, (int)sizeof(T));
+    auto put = [&](auto* to, auto v) {
+      if (alone)
+        *to = v;
+      else
+        st_team(to, v);
+    };
+    for (int g = tg0 + wid; g <= tg1; g += kWaves) {  // one part per wavefront at a time
+      const int32_t p0 = max(row0, aggp[g]), p1 = min(row1, aggp[g + 1]);
+      double m[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) m[c] = 0.0;
+      for (int32_t i = p0 + wl; i < p1; i += 64) {
+        const int l = i - wr0, bits_ = fb[l];
+        double rv[D];
+#pragma unroll
+        for (int e = 0; e < D; ++e) rv[e] = ((bits_ >> e) & 1) ? 0.0 : (double)wl_[l * D + e];
+        if constexpr (D == 3) {
+          const double x = xl[l * 3], y = xl[l * 3 + 1], z = xl[l * 3 + 2];
+          m[0] += rv[0];
+          m[1] += rv[1];
+          m[2] += rv[2];
+          m[3] += y * rv[2] - z * rv[1];
+          m[4] += z * rv[0] - x * rv[2];
+          m[5] += x * rv[1] - y * rv[0];
+        } else if constexpr (D == 2) {
+          m[0] += rv[0];
+          m[1] += rv[1];
+          m[2] += (double)xl[l * 3] * rv[1] - (double)xl[l * 3 + 1] * rv[0];
+        } else {
+          m[0] += rv[0];
+        }
+      }
+      double mine_c = 0.0;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const double t = wave_sum(m[c]);
+        mine_c = wl == c ? t : mine_c;
+      }
+      if (wl < NC) put((T*)(mine + kTeamDots) + (tile + g - q0) * NC + wl, (T)mine_c);
+    }
+    if (dots && threadIdx.x < 3) {
+      double t = 0.0;
+#pragma unroll
+      for (int sb = 0; sb < S; ++sb)
+#pragma unroll
+        for (int q = 0; q < kWaves; ++q) t += s_red[sb][threadIdx.x][q];
+      put((double*)mine + threadIdx.x, t);
+    }
+    if (alone) {
+      __syncthreads();
+    } else {
+      arrive();
+      for (int g = threadIdx.x; g < nwg; g += NT)
+        if (!team_poll(a.abort, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
+      __syncthreads();
+      if (turn == 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the ring's first region, also the first time
+    }
+    if (dots && sub == 0) {
+      double e[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        e[k] = tid < nwg ? ((const double*)(region + team_part(tid, s_q0[tid], NC, (int)sizeof(T))))[k] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        e[k] = wave_sum(e[k]);
+        if (wl == 0) s_sum[k][wid] = e[k];
+      }
+    }
+    // the parts t + g of the tiles t that touch aggregate g
+    for (int e = threadIdx.x; e < n_c; e += NT) {
+      const int g = e / NC, c = e % NC;
+      const int t0 = aggp[g] / R, t1 = min(aggp[g + 1] / R, a.ntiles - 1);
+      double v = 0.0;
+      for (int t = t0; t <= t1; t += kParts) {
+        T part[kParts];
+#pragma unroll
+        for (int j = 0; j < kParts; ++j) {
+          const int tj = min(t + j, t1), q = s_q0[tj / S];
+          part[j] = ((const T*)(region + team_part(tj / S, q, NC, (int)sizeof(T)) + kTeamDots))[(tj + g - q) * NC + c];
+        }
+#pragma unroll
+        for (int j = 0; j < kParts; ++j) v += t + j <= t1 ? (double)part[j] : 0.0;
+      }
+      cm[e] = v;
+    }
+    __syncthreads();
+    return s_fail == 0;
+  };
+  // (behind a barrier) out = B c for the workgroup's aggregates, one wavefront per row
+  auto coarse_apply_rows = [&](double* out) {
+    for (int q = (int)threadIdx.x / 64; q < ng * NC; q += NT / 64) {
+      const T* row = Brows + q * ldb;
+      double v = 0.0;
+#pragma unroll 8
+      for (int c = wl; c < n_c; c += 64) v += (double)row[c] * cm[c];
+      v = wave_sum(v);
+      if (wl == 0) out[q] = v;
+    }
+  };
+  // out = B P^T v, a meeting of its own (reliable updates)
+  auto coarse_round = [&](const T* v, double* out) {
+    coarse_rows(v);
+    __syncthreads();
+    if (!coarse_meet(false)) return false;
+    coarse_apply_rows(out);
+    __syncthreads();
+    return s_fail == 0;
+  };
+  // u += the rigid-body motion z of the node's aggregate, on free DOFs
+  auto coarse_add = [&]() {
+#pragma unroll
+    for (int ps = 0; ps < kPasses; ++ps) {
+      if (la[ps] < 0) continue;
+      const int l = team_here(my_row) + ps * kRows - wr0;
+      const double* y = zc + la[ps];
+      double du = y[lane];
+      if constexpr (D == 3) {
+        // lane 0: z w_y - y w_z, lane 1: x w_z - z w_x, lane 2: y w_x - x w_y
+        const int n1 = lane == 2 ? 0 : lane + 1, n2 = lane == 0 ? 2 : lane - 1;
+        du += (double)xl[l * 3 + n2] * y[3 + n1] - (double)xl[l * 3 + n1] * y[3 + n2];
+      } else if constexpr (D == 2) {
+        du += lane == 0 ? -(double)xl[l * 3 + 1] * y[2] : (double)xl[l * 3] * y[2];
+      }
+      uk[ps] += (T)du;
+    }
+  };
+
   int64_t chunks = 0;
   bool alive = fits;
   while (alive) {
@@ -471,7 +779,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
       for (int ps = 0; ps < kPasses; ++ps) {
         int64_t k;
-        if (own(ps, k)) st_team(a.x + k, xk[ps]);
+        if (own(ps, k)) st_team(a.x + caller(ps, k), xk[ps]);
       }
       if (!meet_neighbours()) { alive = false; break; }
       double v1[1] = {0.0};
@@ -480,7 +788,8 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
         double acc[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) acc[d] = 0.0;
-        for (int32_t q = a.bptr[i] + lane_it; q < a.bptr[i + 1]; q += G) {
+        const int64_t node = CO ? a.order[i] : i;
+        for (int32_t q = a.bptr[node] + lane_it; q < a.bptr[node + 1]; q += G) {
           const int64_t j = a.bcol[q];
           double xj[D];
 #pragma unroll
@@ -496,7 +805,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
         in_registers(acc);
         if (lane_it < D) {
           const int64_t k = (int64_t)i * D + lane_it;
-          const double ri = a.b[k] - pick<double, D>(acc, lane_it);
+          const double ri = a.b[node * D + lane_it] - pick<double, D>(acc, lane_it);
           a.r64[k] = ri;
           v1[0] += ri * ri;
         }
@@ -513,7 +822,11 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
         rk[ps] = (T)a.r64[k];
         if (first) pk[ps] = sk[ps] = T(0);
       }
+      if constexpr (CO) {
+        if (!coarse_round(rk, zc)) { alive = false; break; }
+      }
       precond();
+      if constexpr (CO) coarse_add();
 #pragma unroll
       for (int ps = 0; ps < kPasses; ++ps) {
         int64_t k;
@@ -577,12 +890,22 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
         wk[ps] = w[k];
         sk[ps] = s[k];
       }
+      if constexpr (CO) {
+        if (!coarse_round(wk, yc) || !coarse_round(sk, ze)) { alive = false; break; }
+      }
     }
     // ---- a chunk of iterations ----------------------------------------------------------------------
     if (st.done || ++chunks > a.max_chunks) break;
     for (int it = 0; it < a.chunk; ++it) {
       const double alpha = st.alpha;
       const T alpha_t = (T)alpha, beta = (T)st.beta;
+      if constexpr (CO) {
+        for (int q = threadIdx.x; q < ng * NC; q += NT) {
+          ze[q] = yc[q] + st.beta * ze[q];
+          zc[q] -= alpha * ze[q];
+        }
+        __syncthreads();
+      }
 #pragma unroll
       for (int ps = 0; ps < kPasses; ++ps) {
         pk[ps] = uk[ps] + beta * pk[ps];
@@ -591,6 +914,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
         rk[ps] = rk[ps] - alpha_t * sk[ps];
       }
       precond();
+      if constexpr (CO) coarse_add();
       if (!exchange_u(uk)) { alive = false; break; }
       double v3[3] = {0.0, 0.0, 0.0};
 #pragma unroll
@@ -645,8 +969,28 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
           v3[2] += rd * rd;
         }
       }
-      if (!exchange_dots(v3)) { alive = false; break; }
-      if (threadIdx.x == 0) cg_scalars(&st, cg_in(&st), v3, it == a.chunk - 1);
+      if constexpr (CO) {
+        coarse_rows(wk);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          v3[k] = wave_sum(v3[k]);
+          if (wl == 0) s_red[sub][k][wid] = v3[k];
+        }
+        __syncthreads();
+        if (!coarse_meet(true)) { alive = false; break; }
+        if (threadIdx.x == 0) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            v3[k] = 0.0;
+            for (int q = 0; q < kWaves; ++q) v3[k] += s_sum[k][q];
+          }
+          cg_scalars(&st, cg_in(&st), v3, it == a.chunk - 1);
+        }
+        coarse_apply_rows(yc);
+      } else {
+        if (!exchange_dots(v3)) { alive = false; break; }
+        if (threadIdx.x == 0) cg_scalars(&st, cg_in(&st), v3, it == a.chunk - 1);
+      }
       __syncthreads();
       if (st.done || st.need_ru) break;
     }
@@ -656,7 +1000,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
   for (int ps = 0; ps < kPasses; ++ps) {
     int64_t k;
-    if (own(ps, k)) a.x[k] = xk[ps];
+    if (own(ps, k)) a.x[caller(ps, k)] = xk[ps];
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.st = st;
 }

@@ -380,6 +380,20 @@ class DeviceGraph:
         return self.wmaps
 
 
+def order_pattern(bptr: np.ndarray, bcol: np.ndarray, order: np.ndarray):
+    """(bptr, bcol, src_block) of the pattern whose row and column i are row and column order[i] of the given
+    one; a row's blocks keep their sequence and src_block[q] is block q in the given pattern."""
+    order = np.asarray(order, dtype=np.int64)
+    bptr = np.asarray(bptr, dtype=np.int64)
+    new = np.empty(order.size, dtype=np.int32)
+    new[order] = np.arange(order.size, dtype=np.int32)
+    deg = np.diff(bptr)[order]
+    optr = np.zeros(order.size + 1, dtype=np.int64)
+    optr[1:] = np.cumsum(deg)
+    src = np.repeat(bptr[:-1][order] - optr[:-1], deg) + np.arange(int(optr[-1]), dtype=np.int64)
+    return optr, new[np.asarray(bcol)[src]], src
+
+
 def pad_pattern(bptr: np.ndarray, bcol: np.ndarray, align: int = 4):
     """(bptr, bcol, src_block) of the padded pattern: every block row extended to a multiple of
     ``align`` blocks by blocks whose column is the row itself; src_block[q] is the original block of
@@ -409,16 +423,30 @@ class PaddedGraph:
 
     row_align = 4
 
-    def __init__(self, graph: DeviceGraph):
+    def __init__(self, graph: DeviceGraph, order: Optional[np.ndarray] = None):
         a = self.row_align
         self.ctx = graph.ctx
         self.base = graph
         self.n_nodes = graph.n_nodes
-        pptr, bcol, src = pad_pattern(graph.pattern.bptr, graph.pattern.bcol, a)
+        self.order = order
+        if order is None:
+            pptr, bcol, src = pad_pattern(graph.pattern.bptr, graph.pattern.bcol, a)
+        else:
+            optr, ocol, osrc = order_pattern(graph.pattern.bptr, graph.pattern.bcol, order)
+            pptr, bcol, src = pad_pattern(optr, ocol, a)
+            src[src >= 0] = osrc[src[src >= 0]]
         self.nnzb = int(pptr[-1])
         self.bptr = self.ctx.tensor(pptr)
         self.bcol = self.ctx.tensor(bcol)
         self.src_block = self.ctx.tensor(src)
+
+
+def ordered_graph(graph, order: np.ndarray) -> PaddedGraph:
+    """The graph's padded pattern with node order[i] as its row and column i; the graph keeps the last one."""
+    kept = getattr(graph, '_ordered', None)
+    if kept is None or not np.array_equal(kept.order, order):
+        kept = graph._ordered = PaddedGraph(graph, order)
+    return kept
 
 
 @dataclass
@@ -443,9 +471,10 @@ class BsrMatrix:
                           getattr(self.graph, 'row_align', 0), _vp(self.graph.bptr),
                           _vp(self.graph.bcol), _vp(self.vals))
 
-    def padded(self, dtype=torch.float64) -> 'BsrMatrix':
-        """Iteration copy on the padded pattern (FE_LAYOUT_PLANES, row_align 4) in ``dtype``."""
-        pg = self.graph.padded()
+    def padded(self, dtype=torch.float64, order: Optional[np.ndarray] = None) -> 'BsrMatrix':
+        """Iteration copy on the padded pattern (FE_LAYOUT_PLANES, row_align 4) in ``dtype``; with
+        ``order``, its row and column i are node order[i]."""
+        pg = self.graph.padded() if order is None else ordered_graph(self.graph, order)
         out = BsrMatrix(pg, torch.empty(pg.nnzb * self.dof * self.dof, dtype=dtype,
                                         device=self.vals.device), self.dof, _hip.FE_LAYOUT_PLANES)
         a, b = self.struct(), out.struct()
@@ -759,12 +788,17 @@ class PcgSolver:
         self.M64 = M64
         # the iteration matrix: a copy on the padded pattern (16-byte loads in the SpMV), FP32 with
         # mixed precision; A64 keeps the true residual
-        if self.mixed:
-            self.A32 = A64.padded(torch.float32) if A32 is None else A32
-            self.M32 = _to_f32(self.ctx, self.M64)
-        else:
-            self.A32 = A64.padded(torch.float64) if A32 is None else A32
-            self.M32 = None
+        # a two-level solve that fits on the chip takes it in the order of the aggregates
+        # (fe_pcg_coarse_ordered)
+        self.ordered = False
+        if coarse is not None and segments is None and A32 is None:
+            yes = ctypes.c_int()
+            _hip.call('fe_pcg_coarse_takes_ordered', ctypes.byref(A64.struct()), ctypes.byref(coarse.struct()),
+                      ctypes.byref(self._opts(1e-8, 1)), ctypes.byref(yes))
+            self.ordered = bool(yes.value)
+        order = coarse.host.agg_nodes if self.ordered else None
+        self.A32 = A64.padded(torch.float32 if self.mixed else torch.float64, order) if A32 is None else A32
+        self.M32 = _to_f32(self.ctx, self.M64) if self.mixed else None
         if coarse is not None:
             self.ctx.stream.wait_event(coarse_done)
             for t in (self.Ainv64, self.Ainv32):
@@ -799,7 +833,11 @@ class PcgSolver:
             x = torch.zeros_like(b)
         opts = self._opts(tol, max_iter, profile)
         a64 = self.A64.struct()
-        a32 = self.A32.struct() if self.A32 is not None else None
+        ordered = self.ordered and not profile
+        it = self.A32
+        if self.ordered and profile:  # the profiled kernels are the launched ones, in the mesh's order
+            it = self.A64.padded(torch.float32 if self.mixed else torch.float64)
+        a32 = it.struct() if it is not None else None
         nbytes = ctypes.c_int64()
         cstruct = self.coarse.struct() if self.coarse is not None else None
         if self.segments is not None:
@@ -822,7 +860,11 @@ class PcgSolver:
         stats = _hip.FePcgStats()
         a32p = ctypes.byref(a32) if a32 is not None else None
         seg_info = None
-        if cstruct is not None and self.segments is None:
+        if ordered:
+            _hip.call('fe_pcg_coarse_ordered', ctx.h, ctypes.byref(a64), a32p, _vp(self.M64), _vp(self.M32),
+                      ctypes.byref(cstruct), _vp(self.Ainv64), _vp(b), _vp(x), _vp(self._work),
+                      self._work.numel(), ctypes.byref(opts), ctypes.byref(stats))
+        elif cstruct is not None and self.segments is None:
             _hip.call('fe_pcg_coarse', ctx.h, ctypes.byref(a64), a32p, _vp(self.M64), _vp(self.M32),
                       ctypes.byref(cstruct), _vp(self.Ainv64), _vp(self.Ainv32), _vp(b), _vp(x),
                       _vp(self._work), self._work.numel(), ctypes.byref(opts), ctypes.byref(stats))

@@ -443,6 +443,17 @@ int fe_pcg_coarse_workspace(fe_handle* h, const fe_bsr* A, const fe_coarse* C, c
 int fe_pcg_coarse(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64, const void* M32,
                   const fe_coarse* C, const void* Ainv64, const void* Ainv32, const double* b, double* x,
                   void* work, int64_t work_bytes, const fe_pcg_opts* opts, fe_pcg_stats* stats);
+/* fe_pcg_coarse for a system that fits on the chip, its whole solve in one launch.  Aord: the iteration
+   matrix (FP32 for opts->mixed, else FP64) on a padded pattern (row_align 4) whose row and column i are the
+   node C->agg_nodes[i]; everything else is in the caller's numbering.  Workspace as for fe_pcg_coarse.
+   fe_pcg_coarse_takes_ordered: *yes is 1 for the systems it takes (size, precision, coarse space and
+   options; no GPU needed), FE_ERR_ARG from fe_pcg_coarse_ordered for the others.  A solve that the launch
+   does not end (no co-residency, columns beyond a workgroup's LDS) is finished in FP64 by fe_pcg_coarse's
+   kernels on A64. */
+int fe_pcg_coarse_takes_ordered(const fe_bsr* A, const fe_coarse* C, const fe_pcg_opts* opts, int* yes);
+int fe_pcg_coarse_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
+                          const void* M32, const fe_coarse* C, const void* Ainv64, const double* b, double* x,
+                          void* work, int64_t work_bytes, const fe_pcg_opts* opts, fe_pcg_stats* stats);
 int fe_pcg_batched_coarse_workspace(fe_handle* h, const fe_bsr* A, int32_t n_seg, const int32_t* seg_nodes,
                                     const fe_coarse* C, const fe_pcg_opts* opts, int64_t* bytes);
 int fe_pcg_batched_coarse(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64,

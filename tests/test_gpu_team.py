@@ -122,3 +122,61 @@ def test_team_statuses(ctx):
     solver = s.solver(KD, 'jacobi', 'fp64', M64=device.precond_setup(KD, 'jacobi').abs())
     _, info = solver.solve(b)
     assert info['status'] == _hip.FE_ERR_BREAKDOWN
+
+
+# (kind, size, shuffled, nodes per aggregate): many aggregates in a tile, aggregates as long as a tile (their
+# ends meet), tiles inside one aggregate, one tile, one workgroup of two tiles, several workgroup shapes
+COARSE = [('tet_elastic', 3, False, 8), ('tet_elastic', 5, True, 30), ('tet_elastic', 7, False, 128),
+          ('tet_elastic', 13, True, 1000), ('tet_elastic', 27, True, None), ('tet_elastic', 33, False, None),
+          ('tri_magnetic', (15, 15), False, 256), ('tri_magnetic', (31, 17), True, 20),
+          ('tri_magnetic', (127, 127), False, 256), ('tri_magnetic', (300, 300), False, None),
+          ('tri_elastic', (9, 4), False, 12), ('tri_elastic', (40, 10), True, 81),
+          ('tri_elastic', (120, 50), False, None), ('tri_elastic', (400, 200), False, None),
+          ('tri_magnetic', (400, 400), True, None)]
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('kind,size,shuffled,target', COARSE)
+def test_team_two_level(ctx, kind, size, shuffled, target, precision):
+    """The two-level solve in the order of the aggregates: it reaches the tolerance on the true residual,
+    in the launched kernels' iterations (the correction is carried by recurrence, so not bit for bit), and
+    a second solve by the same solver gives the same bits."""
+    print(f'team two-level {kind} {size} {shuffled} {target} {precision}', flush=True)
+    s, fixed, rng = _problem(kind, size, shuffled)
+    mask, g = s.dirichlet(fixed)
+    coarse = s.coarse_space(fixed, target=target)
+    KD, b = s.prepare(s.stiffness_bsr(), mask, g, ctx.tensor(rng.standard_normal(s.n)), coarse=coarse)
+    solver = s.solver(KD, 'two_level', precision, coarse=coarse)
+    assert solver.ordered
+    tol = 1e-9
+    u, info = solver.solve(b, tol=tol)
+    assert info['status'] == 0 and info['relres'] <= tol and info['fallbacks'] == 0
+    res = b - device.spmv(KD, u)
+    assert float(res.norm()) <= 1.001 * tol * float(b.norm())
+    _, launched = solver.solve(b, tol=tol, profile=True)
+    assert launched['status'] == 0
+    assert abs(info['iterations'] - launched['iterations']) <= 16 + launched['iterations'] // 8
+    u2, info2 = solver.solve(b, tol=tol)
+    assert info2['iterations'] == info['iterations'] and torch.equal(u, u2)
+    # a start that already solves the system needs no iteration, and keeps its bits
+    x, info = solver.solve(b, x=u.clone(), tol=2 * tol)
+    assert info['iterations'] == 0 and torch.equal(x, u)
+
+
+def test_team_two_level_beyond_its_sizes(ctx):
+    """FP64 beyond 512 tiles and a coarse space beyond its limit go to the launched kernels."""
+    print('team two-level limits', flush=True)
+    s, fixed, _ = _problem('tet_elastic', 41)
+    mask, g = s.dirichlet(fixed)
+    coarse = s.coarse_space(fixed)
+    KD, b = s.prepare(s.stiffness_bsr(), mask, g, ctx.zeros(s.n), coarse=coarse)
+    assert not s.solver(KD, 'two_level', 'fp64', coarse=coarse).ordered
+    assert s.solver(KD, 'two_level', 'mixed', coarse=coarse).ordered
+    s, fixed, rng = _problem('tri_magnetic', (60, 60))
+    mask, g = s.dirichlet(fixed)
+    coarse = s.coarse_space(fixed, target=2)
+    assert coarse.n_coarse > 1536
+    KD, b = s.prepare(s.stiffness_bsr(), mask, g, ctx.tensor(rng.standard_normal(s.n)), coarse=coarse)
+    solver = s.solver(KD, 'two_level', 'fp64', coarse=coarse)
+    assert not solver.ordered
+    assert solver.solve(b, tol=1e-9)[1]['status'] == 0

@@ -8,10 +8,9 @@
 //   K2 k_lob_spmm    K W and M W in one pass over the shared pattern
 //   K3 k_lob_gram    partial Gram matrices S^T K S, S^T M S of the basis S = [X W P]
 //   K4 k_lob_gsum    fixed-order sum of the partials
-//   K5 k_lob_rr      one workgroup: convergence test, then Rayleigh-Ritz with a rank-revealing
-//                    M-orthonormalisation of S (eigen-decomposition of the scaled S^T M S, directions
-//                    below a relative threshold dropped), both small eigenproblems by parallel cyclic
-//                    Jacobi in LDS
+//   K5 k_lob_rr      one workgroup: convergence test, then Rayleigh-Ritz with a rank-checked
+//                    M-orthonormalisation of S (Cholesky of the scaled S^T M S, columns with a pivot
+//                    below a threshold dropped); the small eigenproblem by parallel cyclic Jacobi in LDS
 //   K6 k_lob_update_rows X' = S C, P' = [W P] C_WP, with the K- and M-images recombined the same way
 //   K7 k_lob_flip    swap the double-buffered blocks, advance the iteration
 // Block vectors are stored row-major [n][m] (the m columns of one DOF row contiguous), so every
@@ -138,8 +137,8 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid(LobParams p, const doubl
 // one aggregate), forming R, W = T R and the column norms as k_lob_resid does and r_c = P^T R (thread
 // (group g, column j) sums an aggregate's nodes g, g + npg, ..., then the groups are added in a
 // fixed order), so K X and M X are read once per iteration.
-template <int D, int NC>
-__global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coarse C, int64_t ld,
+template <int D, int NC, int NT>
+__global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, int64_t ld,
                                                             const double* __restrict__ T, int64_t t_stride,
                                                             const uint8_t* __restrict__ fixed,
                                                             const LobState* st, double* blk,
@@ -149,8 +148,8 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coar
   __shared__ int s_skip, s_cur;
   __shared__ double s_lam[kMaxBlock];
   __shared__ int s_lock[kMaxBlock];
-  __shared__ double s_rr[kThreads], s_bb[kThreads];
-  __shared__ double s_acc[kThreads][NC];
+  __shared__ double s_rr[NT], s_bb[NT];
+  __shared__ double s_acc[NT][NC];
   if (threadIdx.x == 0) {
     s_skip = st[v].done;
     s_cur = st[v].cur;
@@ -163,13 +162,14 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coar
   __syncthreads();
   if (s_skip) return;
   const int m = p.m;
-  const int npg = kThreads / m;
+  const int npg = NT / m;
   const int g = threadIdx.x / m, j = threadIdx.x % m;
   const double* KX = lob_block(blk, p, v, B_KX + s_cur);
   const double* MX = lob_block(blk, p, v, B_MX + s_cur);
   double* W = lob_block(blk, p, v, B_W);
   const double* Tv = T ? T + (int64_t)v * t_stride : nullptr;
   const int64_t alo = C.n_agg * blockIdx.x / gridDim.x, ahi = C.n_agg * (blockIdx.x + 1) / gridDim.x;
+  double* out = rpart + ((int64_t)v * gridDim.x + blockIdx.x) * 2 * m;
   const double lam = s_lam[j];
   double rr = 0.0, bb = 0.0;
   for (int64_t agg = alo; agg < ahi; ++agg) {
@@ -208,26 +208,41 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coar
 #pragma unroll
     for (int c = 0; c < NC; ++c) s_acc[threadIdx.x][c] = acc[c];
     __syncthreads();
-    if (threadIdx.x < m * NC) {
-      const int jj = threadIdx.x % m, c = threadIdx.x / m;
+    // the groups' sums over `ways` threads each (groups way, way + ways, ...), then those in order
+    const int outs = m * NC, ways = NT / outs, way = threadIdx.x / outs;
+    if (way < ways) {
+      const int jj = threadIdx.x % m, c = threadIdx.x % outs / m;
       double sum = 0.0;
-      for (int q = 0; q < npg; ++q) sum += s_acc[q * m + jj][c];
-      rc[((int64_t)v * ld + agg * NC + c) * m + jj] = sum;
+#pragma unroll 4
+      for (int q = way; q < npg; q += ways) sum += s_acc[q * m + jj][c];
+      s_rr[threadIdx.x] = sum;
     }
     __syncthreads();
+    if (threadIdx.x < outs) {
+      double sum = s_rr[threadIdx.x];
+      for (int q = 1; q < ways; ++q) sum += s_rr[q * outs + threadIdx.x];
+      rc[((int64_t)v * ld + agg * NC + threadIdx.x / m) * m + threadIdx.x % m] = sum;
+    }
   }
+  __syncthreads();
+  // column norms, the same way: outputs x < m are R's, the others M X's
+  double* const s_nn = &s_acc[0][0];
   s_rr[threadIdx.x] = rr;
   s_bb[threadIdx.x] = bb;
   __syncthreads();
-  if (threadIdx.x < m) {
-    double a = 0.0, b = 0.0;
-    for (int q = 0; q < npg; ++q) {
-      a += s_rr[q * m + threadIdx.x];
-      b += s_bb[q * m + threadIdx.x];
-    }
-    double* out = rpart + ((int64_t)v * gridDim.x + blockIdx.x) * 2 * m;
-    out[threadIdx.x] = a;
-    out[m + threadIdx.x] = b;
+  const int outs = 2 * m, ways = NT / outs, way = threadIdx.x / outs, x = threadIdx.x % outs;
+  if (way < ways) {
+    const double* src = x < m ? s_rr + x : s_bb + x - m;
+    double sum = 0.0;
+#pragma unroll 4
+    for (int q = way; q < npg; q += ways) sum += src[q * m];
+    s_nn[threadIdx.x] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x < outs) {
+    double sum = s_nn[threadIdx.x];
+    for (int q = 1; q < ways; ++q) sum += s_nn[q * outs + threadIdx.x];
+    out[threadIdx.x] = sum;
   }
 }
 
@@ -638,6 +653,27 @@ __global__ __launch_bounds__(kGramThreads, 2) void k_lob_gram(LobParams p, const
     gram_rows<0>(base, ns, nT, m, bS, bY, p.nm, lo, hi, out, NS);
 }
 
+// Sum of an entry's chunk partials src[0], src[stride], ... over kSumWays threads (chunk k is thread k %
+// kSumWays's, then the threads in order), result in the first.  One thread walking the up to 512 chunks
+// took 127 us at 512 chunks of 4 variants (36 columns); this takes 24.
+constexpr int kSumWays = 16, kSumEntries = kThreads / kSumWays;
+
+__device__ inline double chunk_sum(const double* __restrict__ src, int64_t stride, int n, bool live) {
+  __shared__ double part[kSumWays][kSumEntries + 1];
+  const int e = threadIdx.x % kSumEntries, way = threadIdx.x / kSumEntries;
+  double g = 0.0;
+  if (live) {
+#pragma unroll 8
+    for (int k = way; k < n; k += kSumWays) g += src[(int64_t)k * stride];
+  }
+  part[way][e] = g;
+  __syncthreads();
+  if (way != 0) return 0.0;
+#pragma unroll
+  for (int w = 1; w < kSumWays; ++w) g += part[w][e];
+  return g;
+}
+
 // K4: fixed-order sum of the Gram partials into G[v][2][NS][NS] (both triangles).
 __global__ __launch_bounds__(kThreads) void k_lob_gsum(LobParams p, const LobState* st,
                                                        const double* __restrict__ gpart,
@@ -645,17 +681,15 @@ __global__ __launch_bounds__(kThreads) void k_lob_gsum(LobParams p, const LobSta
   const int v = blockIdx.y;
   if (st[v].done) return;
   const int NS = 3 * p.m, ns = st[v].ns;
-  const int e = blockIdx.x * kThreads + threadIdx.x;
-  if (e >= 2 * NS * NS) return;
+  const int e = blockIdx.x * kSumEntries + threadIdx.x % kSumEntries;
   const int mat = e / (NS * NS), a = (e % (NS * NS)) / NS, b = e % NS;
-  if (a >= ns || b >= ns) return;
+  const bool live = e < 2 * NS * NS && a < ns && b < ns;
   // below the diagonal only the diagonal tiles hold entries; elsewhere read the upper entry
   const int at = a / kGramTile, bt = b / kGramTile;
   const int ra = (at > bt) ? b : a, rb = (at > bt) ? a : b;
-  double s = 0.0;
-  const double* src = gpart + (int64_t)v * p.nchunk_g * 2 * NS * NS + mat * NS * NS + ra * NS + rb;
-  for (int c = 0; c < p.nchunk_g; ++c) s += src[(int64_t)c * 2 * NS * NS];
-  G[((int64_t)v * 2 + mat) * NS * NS + a * NS + b] = s;
+  const double s = chunk_sum(gpart + (int64_t)v * p.nchunk_g * 2 * NS * NS + mat * NS * NS + ra * NS + rb,
+                             2 * NS * NS, p.nchunk_g, live);
+  if (live && threadIdx.x < kSumEntries) G[((int64_t)v * 2 + mat) * NS * NS + a * NS + b] = s;
 }
 
 // --------------------------------------------------------------------------------------------------
@@ -763,18 +797,15 @@ __global__ __launch_bounds__(kThreads) void k_lob_gsum_w(LobParams p, const LobS
   const int v = blockIdx.y;
   if (st[v].done) return;
   const int m = p.m, NS = 3 * m, ns = st[v].ns;
-  const int e = blockIdx.x * kThreads + threadIdx.x;
-  if (e >= 2 * NS * NS) return;
+  const int e = blockIdx.x * kSumEntries + threadIdx.x % kSumEntries;
   const int mat = e / (NS * NS), a = (e % (NS * NS)) / NS, b = e % NS;
-  if (a >= ns || b >= ns) return;
+  const bool live = e < 2 * NS * NS && a < ns && b < ns;
   const bool aw = a >= m && a < 2 * m, bw = b >= m && b < 2 * m;
-  double g;
-  if (aw || bw) {
-    const int r = bw ? a : b, c = bw ? b - m : a - m;  // (row of S, column of W)
-    const double* src = gpart + ((int64_t)v * p.nchunk_g * 2 + mat) * NS * m + r * m + c;
-    g = 0.0;
-    for (int k = 0; k < p.nchunk_g; ++k) g += src[(int64_t)k * 2 * NS * m];
-  } else {
+  const int r = bw ? a : b, c = bw ? b - m : a - m;  // (row of S, column of W)
+  double g = chunk_sum(gpart + ((int64_t)v * p.nchunk_g * 2 + mat) * NS * m + r * m + c, 2 * NS * m, p.nchunk_g,
+                       live && (aw || bw));
+  if (!live || threadIdx.x >= kSumEntries) return;
+  if (!aw && !bw) {
     const int ia = a < m ? a : a - m, ib = b < m ? b : b - m;  // X: 0..m-1, P: m..2m-1
     const int lo_ = ia < ib ? ia : ib, hi_ = ia < ib ? ib : ia;
     g = Gp[(((int64_t)v * 2 + mat) * 2 * m + lo_) * 2 * m + hi_];
@@ -786,108 +817,143 @@ __global__ __launch_bounds__(kThreads) void k_lob_gsum_w(LobParams p, const LobS
 // Parallel cyclic Jacobi on an r x r symmetric matrix in LDS (row-major, leading dimension r).
 // On return the diagonal of A holds the eigenvalues and the columns of V the eigenvectors.
 // Round-robin pairing: every step rotates r/2 disjoint planes at once (rows, then columns).
+//
+// Bound by the latency of a step (about ten sweeps of r - 1 dependent steps on one workgroup), so: the
+// rotations of a step are formed by the first wavefront while the others apply the previous step's to V;
+// angles take two reciprocal square roots instead of two roots and three divisions; work items map to
+// threads without divisions.  The whole Rayleigh-Ritz kernel went from 875 to 267 us at 36 columns (the
+// Cholesky below and products from LDS included); 512 threads make a modal run of that size 8% slower.
 // --------------------------------------------------------------------------------------------------
+// 1 / sqrt(x) for a positive normal x: the hardware's estimate and two Newton steps.
+__device__ inline double fast_rsqrt(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = y * (1.5 - 0.5 * x * y * y);
+  return y * (1.5 - 0.5 * x * y * y);
+}
+
+// Rotation (c, s) that diagonalises [[app, apq], [apq, aqq]], of the smaller angle.
+__device__ inline void jacobi_angle(double app, double aqq, double apq, double& c, double& s) {
+  c = 1.0;
+  s = 0.0;
+  double d = aqq - app, h = 2.0 * apq;
+  const double big = fmax(fabs(d), fabs(h));
+  if (!(big > 0.0) || apq == 0.0) return;  // (a NaN leaves the pair alone)
+  const int e = -__builtin_amdgcn_frexp_exp(big);  // entries far from 1 would leave the range when squared
+  d = ldexp(d, e);
+  h = ldexp(h, e);
+  const double ir = fast_rsqrt(d * d + h * h);
+  const double x = 0.5 + 0.5 * fabs(d) * ir;  // cos^2
+  const double ic = fast_rsqrt(x);
+  c = x * ic;
+  s = (d >= 0.0 ? 0.5 : -0.5) * h * ir * ic;
+}
+
 // Stops when the off-diagonal squared norm is at most off2 times the diagonal's.
 __device__ void jacobi_eig(double* A, double* V, int r, int max_sweeps, double off2 = 1e-30) {
-  __shared__ double s_c[kMaxBasis / 2 + 1], s_s[kMaxBasis / 2 + 1];
-  __shared__ int s_p[kMaxBasis / 2 + 1], s_q[kMaxBasis / 2 + 1];
+  __shared__ double s_c[2][kMaxBasis / 2], s_s[2][kMaxBasis / 2];
+  __shared__ int s_p[2][kMaxBasis / 2], s_q[2][kMaxBasis / 2];
   __shared__ double s_off[kRRThreads / 64], s_dia[kRRThreads / 64];
-  __shared__ int s_stop;
-  const int tid = threadIdx.x, nth = blockDim.x;
+  const int tid = threadIdx.x, nth = blockDim.x, wave = tid >> 6, nwaves = nth >> 6;
   for (int idx = tid; idx < r * r; idx += nth) V[idx] = (idx / r == idx % r) ? 1.0 : 0.0;
   const int re = r + (r & 1), npair = re / 2;
+  // a work item's pair in the low bits of the thread index (32 or 64 pairs)
+  const int lbits = npair <= 32 ? 5 : 6, l = tid & ((1 << lbits) - 1), k0 = tid >> lbits, kstep = nth >> lbits;
+  // pair t of a step: 0 meets re - 1 - step, the others turn around it
+  auto place = [&](int i, int step) {
+    int at = i - 1 + step;
+    if (at >= re - 1) at -= re - 1;
+    return i == 0 ? 0 : at + 1;
+  };
+  auto rotations = [&](int step, int buf) {  // the first wavefront
+    if (tid >= npair) return;
+    int p = place(tid, step), q = place(re - 1 - tid, step);
+    if (p > q) {
+      const int t = p;
+      p = q;
+      q = t;
+    }
+    double c = 1.0, s = 0.0;
+    if (q < r) jacobi_angle(A[p * r + p], A[q * r + q], A[p * r + q], c, s);
+    s_p[buf][tid] = p;
+    s_q[buf][tid] = q;
+    s_c[buf][tid] = c;
+    s_s[buf][tid] = s;
+  };
+  auto turn_v = [&](int buf, int k, int kst) {  // columns p, q of V, rows k, k + kst, ...
+    if (l >= npair) return;
+    const int p = s_p[buf][l], q = s_q[buf][l];
+    const double c = s_c[buf][l], s = s_s[buf][l];
+    if (q >= r || s == 0.0) return;
+    for (int i = k; i < r; i += kst) {
+      const double vp = V[i * r + p], vq = V[i * r + q];
+      V[i * r + p] = c * vp - s * vq;
+      V[i * r + q] = s * vp + c * vq;
+    }
+  };
   __syncthreads();
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     double off = 0.0, dia = 0.0;
-    for (int idx = tid; idx < r * r; idx += nth) {
-      const double a = A[idx];
-      if (idx / r == idx % r)
-        dia += a * a;
-      else
-        off += a * a;
-    }
+    for (int i = wave; i < r; i += nwaves)
+      for (int j = tid & 63; j < r; j += 64) {
+        const double a = A[i * r + j];
+        dia += i == j ? a * a : 0.0;
+        off += i == j ? 0.0 : a * a;
+      }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       off += __shfl_xor(off, o, 64);
       dia += __shfl_xor(dia, o, 64);
     }
     if ((tid & 63) == 0) {
-      s_off[tid >> 6] = off;
-      s_dia[tid >> 6] = dia;
+      s_off[wave] = off;
+      s_dia[wave] = dia;
     }
     __syncthreads();
-    if (tid == 0) {
-      double o2 = 0.0, d2 = 0.0;
-      for (int w = 0; w < (nth + 63) / 64; ++w) {
-        o2 += s_off[w];
-        d2 += s_dia[w];
-      }
-      s_stop = !(o2 > off2 * d2);
+    double o2 = 0.0, d2 = 0.0;
+    for (int w = 0; w < nwaves; ++w) {
+      o2 += s_off[w];
+      d2 += s_dia[w];
     }
+    if (!(o2 > off2 * d2)) break;  // uniform
+    rotations(0, 0);
     __syncthreads();
-    if (s_stop) break;
     for (int step = 0; step < re - 1; ++step) {
-      if (tid < npair) {
-        auto pos = [&](int i) { return i == 0 ? 0 : ((i - 1 + step) % (re - 1)) + 1; };
-        int pp = pos(tid), qq = pos(re - 1 - tid);
-        if (pp > qq) {
-          const int t = pp;
-          pp = qq;
-          qq = t;
-        }
-        double c = 1.0, s = 0.0;
-        if (qq < r) {
-          const double apq = A[pp * r + qq];
-          if (apq != 0.0) {
-            const double app = A[pp * r + pp], aqq = A[qq * r + qq];
-            const double tau = (aqq - app) / (2.0 * apq);
-            double t;
-            if (fabs(tau) > 1e150)
-              t = 0.5 / tau;
-            else
-              t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-            c = 1.0 / sqrt(1.0 + t * t);
-            s = t * c;
+      const int buf = step & 1;
+      // A <- J^T A J in one pass: each 2 x 2 block (rows {p_k, q_k}, columns {p_l, q_l}) gets the row
+      // rotation of pair k, then the column rotation of pair l
+      if (l < npair) {
+        const int p2 = s_p[buf][l], q2 = s_q[buf][l];
+        const bool hq2 = q2 < r;
+        const double c2 = s_c[buf][l], s2 = s_s[buf][l];
+        for (int k = k0; k < npair; k += kstep) {
+          const int p1 = s_p[buf][k], q1 = s_q[buf][k];
+          const bool hq1 = q1 < r;
+          const double c1 = s_c[buf][k], s1 = s_s[buf][k];
+          const double a_pp = A[p1 * r + p2], a_pq = hq2 ? A[p1 * r + q2] : 0.0;
+          const double a_qp = hq1 ? A[q1 * r + p2] : 0.0;
+          const double a_qq = (hq1 && hq2) ? A[q1 * r + q2] : 0.0;
+          // rows
+          const double r_pp = c1 * a_pp - s1 * a_qp, r_pq = c1 * a_pq - s1 * a_qq;
+          const double r_qp = s1 * a_pp + c1 * a_qp, r_qq = s1 * a_pq + c1 * a_qq;
+          // columns
+          A[p1 * r + p2] = c2 * r_pp - s2 * r_pq;
+          if (hq2) A[p1 * r + q2] = s2 * r_pp + c2 * r_pq;
+          if (hq1) {
+            A[q1 * r + p2] = c2 * r_qp - s2 * r_qq;
+            if (hq2) A[q1 * r + q2] = s2 * r_qp + c2 * r_qq;
           }
         }
-        s_p[tid] = pp;
-        s_q[tid] = qq;
-        s_c[tid] = c;
-        s_s[tid] = s;
       }
       __syncthreads();
-      // A <- J^T A J in one pass: each 2 x 2 block (rows {p_k, q_k}, columns {p_l, q_l}) gets the row
-      // rotation of pair k, then the column rotation of pair l (the same operations, in the same
-      // order, as rotating all rows and then all columns); V <- V J alongside
-      for (int idx = tid; idx < npair * npair; idx += nth) {
-        const int k = idx / npair, l = idx - k * npair;
-        const int p1 = s_p[k], q1 = s_q[k], p2 = s_p[l], q2 = s_q[l];
-        const bool hq1 = q1 < r, hq2 = q2 < r;
-        const double c1 = s_c[k], s1 = s_s[k], c2 = s_c[l], s2 = s_s[l];
-        const double a_pp = A[p1 * r + p2], a_pq = hq2 ? A[p1 * r + q2] : 0.0;
-        const double a_qp = hq1 ? A[q1 * r + p2] : 0.0;
-        const double a_qq = (hq1 && hq2) ? A[q1 * r + q2] : 0.0;
-        // rows
-        const double r_pp = c1 * a_pp - s1 * a_qp, r_pq = c1 * a_pq - s1 * a_qq;
-        const double r_qp = s1 * a_pp + c1 * a_qp, r_qq = s1 * a_pq + c1 * a_qq;
-        // columns
-        A[p1 * r + p2] = c2 * r_pp - s2 * r_pq;
-        if (hq2) A[p1 * r + q2] = s2 * r_pp + c2 * r_pq;
-        if (hq1) {
-          A[q1 * r + p2] = c2 * r_qp - s2 * r_qq;
-          if (hq2) A[q1 * r + q2] = s2 * r_qp + c2 * r_qq;
-        }
-      }
-      for (int idx = tid; idx < r * npair; idx += nth) {
-        const int k = idx / r, i = idx - k * r;
-        const int qq = s_q[k];
-        const double s = s_s[k];
-        if (qq >= r || s == 0.0) continue;
-        const int pp = s_p[k];
-        const double c = s_c[k];
-        const double vp = V[i * r + pp], vq = V[i * r + qq];
-        V[i * r + pp] = c * vp - s * vq;
-        V[i * r + qq] = s * vp + c * vq;
+      // V <- V J by the wavefronts after the first (which forms the next rotations), or by all at the end
+      const int first = (64 >> lbits);  // rows per pass that the first wavefront would take
+      if (step + 1 < re - 1) {
+        if (wave == 0)
+          rotations(step + 1, buf ^ 1);
+        else
+          turn_v(buf, k0 - first, kstep - first);
+      } else {
+        turn_v(buf, k0, kstep);
       }
       __syncthreads();
     }
@@ -917,6 +983,52 @@ __global__ __launch_bounds__(kRRThreads) void k_sym_eig(int r, const double* __r
   for (int i = threadIdx.x; i < r; i += blockDim.x) w[mat * r + i] = sA[i * r + i];
 }
 
+// C (n x q, leading dimension ldc) = A B, A n x l (TA: A^T, A stored l x n) and B l x q, all in LDS; C may be A
+// or B (every thread holds its outputs until all operands are read).  Three 2 x 2 outputs per thread
+// cover kMaxBasis x kMaxBasis.
+constexpr int kRRItems = kMaxBasis * kMaxBasis / kRRThreads;  // entries of a basis matrix per thread
+static_assert(kRRItems * kRRThreads == kMaxBasis * kMaxBasis, "whole items");
+template <bool TA>
+__device__ void lds_product(int n, int q, int l, const double* A, int lda, const double* B, int ldb, double* C, int ldc) {
+  constexpr int kTiles = (kMaxBasis / 2 * (kMaxBasis / 2) + kRRThreads - 1) / kRRThreads;
+  const int n2 = (n + 1) / 2, q2 = (q + 1) / 2;
+  double acc[kTiles][2][2];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    const int idx = threadIdx.x + t * kRRThreads;
+    if (idx >= n2 * q2) break;
+    const int i = 2 * (idx / q2), j = 2 * (idx % q2);
+    const int i1 = min(i + 1, n - 1), j1 = min(j + 1, q - 1);
+    double c00 = 0.0, c01 = 0.0, c10 = 0.0, c11 = 0.0;
+#pragma unroll 4
+    for (int k = 0; k < l; ++k) {
+      const double a0 = TA ? A[k * lda + i] : A[i * lda + k], a1 = TA ? A[k * lda + i1] : A[i1 * lda + k];
+      const double b0 = B[k * ldb + j], b1 = B[k * ldb + j1];
+      c00 += a0 * b0;
+      c01 += a0 * b1;
+      c10 += a1 * b0;
+      c11 += a1 * b1;
+    }
+    acc[t][0][0] = c00;
+    acc[t][0][1] = c01;
+    acc[t][1][0] = c10;
+    acc[t][1][1] = c11;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    const int idx = threadIdx.x + t * kRRThreads;
+    if (idx >= n2 * q2) break;
+    const int i = 2 * (idx / q2), j = 2 * (idx % q2);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+        if (i + x < n && j + y < q) C[(i + x) * ldc + j + y] = acc[t][x][y];
+  }
+  __syncthreads();
+}
+
 // --------------------------------------------------------------------------------------------------
 // K5: convergence test and Rayleigh-Ritz, one workgroup per variant.
 // --------------------------------------------------------------------------------------------------
@@ -924,7 +1036,6 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
                                                        const double* __restrict__ rpart,
                                                        const double* __restrict__ G,
                                                        double* __restrict__ Zg,
-                                                       double* __restrict__ Tg,
                                                        double* __restrict__ Cg,
                                                        double* __restrict__ Gp) {
   extern __shared__ double lds[];
@@ -935,6 +1046,7 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   __shared__ int s_sel[kMaxBlock];
   __shared__ double s_scale[kMaxBasis];
   __shared__ double s_mu[kMaxBasis];
+  __shared__ double s_norm[2 * kMaxBlock];
   const int m = p.m, NS = 3 * m, tid = threadIdx.x;
   if (tid == 0) {
     s_skip = s->done;
@@ -946,13 +1058,21 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   const int ns = s_ns;
   // ---- convergence of the current block (its residuals were formed by k_lob_resid) ----
   if (!s_init) {
+    // the chunks' norms, 16 threads per column and sum (chunk c is thread c % 16's, then in order)
+    constexpr int kWays = 16;
+    const int way = tid % kWays;
+    for (int col = tid / kWays; col < 2 * m; col += kRRThreads / kWays) {  // column j's: j (residual), m + j
+      double a = 0.0;
+      const double* src = rpart + (int64_t)v * p.nchunk_r * 2 * m + col;
+#pragma unroll 4
+      for (int c = way; c < p.nchunk_r; c += kWays) a += src[(int64_t)c * 2 * m];
+#pragma unroll
+      for (int o = kWays / 2; o > 0; o >>= 1) a += __shfl_xor(a, o, kWays);
+      if (way == 0) s_norm[col] = a;
+    }
+    __syncthreads();
     if (tid < m) {
-      double a = 0.0, b = 0.0;
-      const double* src = rpart + (int64_t)v * p.nchunk_r * 2 * m;
-      for (int c = 0; c < p.nchunk_r; ++c) {
-        a += src[(int64_t)c * 2 * m + tid];
-        b += src[(int64_t)c * 2 * m + m + tid];
-      }
+      const double a = s_norm[tid], b = s_norm[m + tid];
       const double lam = fabs(s->lambda[tid]);
       const double den = (lam > 0.0 ? lam : 1.0) * sqrt(b);
       s->resid[tid] = den > 0.0 ? sqrt(a) / den : sqrt(a);
@@ -976,26 +1096,41 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   const double* GK = G + (int64_t)v * 2 * NS * NS;
   const double* GM = GK + NS * NS;
   double* Z = Zg + (int64_t)v * NS * NS;
-  double* T1 = Tg + (int64_t)v * NS * NS;
-  // ---- rank-revealing M-orthonormalisation of the basis: eig of D GM D, D = diag(GM)^-1/2 ----
+  // ---- M-orthonormalisation of the basis with a rank check: Cholesky of D GM D, D = diag(GM)^-1/2, in the
+  // order X, W, P, dropping a column whose pivot (the squared norm of what its predecessors leave of it)
+  // is at most p.drop.  sA holds the Schur complement, sV the basis change Z: step k takes column k
+  // out of the columns after it, in both.  One barrier per step; the eigen-decomposition that this replaces
+  // took eight to ten sweeps of steps (354 us at r = 36).
   if (tid < ns) {
     const double d = GM[tid * NS + tid];
     s_scale[tid] = d > 0.0 ? 1.0 / sqrt(d) : 0.0;
   }
   __syncthreads();
-  for (int idx = tid; idx < ns * ns; idx += blockDim.x) {
-    const int a = idx / ns, b = idx % ns;
-    sA[idx] = 0.5 * (GM[a * NS + b] + GM[b * NS + a]) * s_scale[a] * s_scale[b];
-  }
+  const int wave = tid >> 6, nwaves = blockDim.x >> 6, lane = tid & 63;
+  for (int a = wave; a < ns; a += nwaves)
+    for (int b = lane; b < ns; b += 64) {
+      sA[a * ns + b] = 0.5 * (GM[a * NS + b] + GM[b * NS + a]) * s_scale[a] * s_scale[b];
+      sV[a * ns + b] = a == b ? 1.0 : 0.0;
+    }
   __syncthreads();
-  jacobi_eig(sA, sV, ns, kJacobiSweeps, kRROff2);
+  for (int k = 0; k < ns; ++k) {
+    const double piv = sA[k * ns + k];
+    if (piv > p.drop) {  // uniform
+      const double inv = 1.0 / piv;
+      for (int j = k + 1 + lane; j < ns; j += 64) {
+        const double f = sA[k * ns + j] * inv;
+        for (int i = k + 1 + wave; i < ns; i += nwaves) sA[i * ns + j] -= sA[k * ns + i] * f;
+        for (int i = wave; i <= k; i += nwaves) sV[i * ns + j] -= sV[i * ns + k] * f;
+      }
+    }
+    __syncthreads();
+  }
   if (tid == 0) {
-    double mx = 0.0;
-    for (int k = 0; k < ns; ++k) mx = fmax(mx, sA[k * ns + k]);
-    int kept = 0;
+    int kept = 0, zero = 0;
     for (int k = 0; k < ns; ++k) {
       const double mu = sA[k * ns + k];
-      if (mu > p.drop * mx) {
+      zero += !(s_scale[k] > 0.0);
+      if (mu > p.drop) {
         s_kept[kept] = k;
         s_mu[kept] = mu;
         ++kept;
@@ -1005,8 +1140,6 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
     s->kept = kept;
     // directions dropped for near-dependence (soft-locked W columns aside): the next iteration
     // restarts the search from [X W] without P
-    int zero = 0;
-    for (int k = 0; k < ns; ++k) zero += !(s_scale[k] > 0.0);
     s->restart = (kept + zero < ns);
   }
   __syncthreads();
@@ -1015,35 +1148,35 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
     if (tid == 0) s->done = 3;
     return;
   }
-  // Z = D Q_kept diag(mu)^-1/2 (ns x rk), leading dimension NS
-  for (int idx = tid; idx < ns * rk; idx += blockDim.x) {
-    const int a = idx / rk, k = idx % rk;
-    Z[a * NS + k] = s_scale[a] * sV[a * ns + s_kept[k]] / sqrt(s_mu[k]);
+  // Z = D L^-T of the kept columns (ns x rk), also in LDS (leading dimension rk); symmetric GK into sA
+  {
+    double z[kRRItems];
+#pragma unroll
+    for (int t = 0; t < kRRItems; ++t) {
+      const int idx = tid + t * kRRThreads;
+      if (idx < ns * rk) {
+        const int a = idx / rk, k = idx - a * rk;
+        z[t] = s_scale[a] * sV[a * ns + s_kept[k]] / sqrt(s_mu[k]);
+        Z[a * NS + k] = z[t];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kRRItems; ++t)
+      if (tid + t * kRRThreads < ns * rk) sV[tid + t * kRRThreads] = z[t];
   }
+  for (int a = wave; a < ns; a += nwaves)
+    for (int b = lane; b < ns; b += 64) sA[a * ns + b] = 0.5 * (GK[a * NS + b] + GK[b * NS + a]);
   __syncthreads();
-  // T1 = GK Z (ns x rk), then H = Z^T T1 (rk x rk) into sA
-  for (int idx = tid; idx < ns * rk; idx += blockDim.x) {
-    const int a = idx / rk, k = idx % rk;
-    double t = 0.0;
-    for (int b = 0; b < ns; ++b) t += 0.5 * (GK[a * NS + b] + GK[b * NS + a]) * Z[b * NS + k];
-    T1[a * NS + k] = t;
-  }
-  __syncthreads();
-  for (int idx = tid; idx < rk * rk; idx += blockDim.x) {
-    const int k = idx / rk, l = idx % rk;
-    double h = 0.0;
-    for (int a = 0; a < ns; ++a) h += Z[a * NS + k] * T1[a * NS + l];
-    sA[idx] = h;
-  }
-  __syncthreads();
-  for (int idx = tid; idx < rk * rk; idx += blockDim.x) {
-    const int k = idx / rk, l = idx % rk;
-    if (k < l) {
+  // H = Z^T (GK Z) (rk x rk) in sA, through registers
+  lds_product<false>(ns, rk, ns, sA, ns, sV, rk, sA, rk);
+  lds_product<true>(rk, rk, ns, sV, rk, sA, rk, sA, rk);
+  for (int k = wave; k < rk; k += nwaves)
+    for (int l = lane; l < k; l += 64) {
       const double h = 0.5 * (sA[k * rk + l] + sA[l * rk + k]);
       sA[k * rk + l] = h;
       sA[l * rk + k] = h;
     }
-  }
   __syncthreads();
   jacobi_eig(sA, sV, rk, kJacobiSweeps, kRROff2);
   // select the m smallest (largest) Ritz values in order: thread k ranks value k (ties by index)
@@ -1061,44 +1194,52 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
     }
   }
   __syncthreads();
-  // C = Z Y_sel (ns x m)
+  // C = Z Y_sel (ns x m): Y_sel and then C in sV, Z in sA
   double* C = Cg + (int64_t)v * NS * m;
-  for (int idx = tid; idx < ns * m; idx += blockDim.x) {
-    const int a = idx / m, j = idx % m;
-    double c = 0.0;
-    for (int k = 0; k < rk; ++k) c += Z[a * NS + k] * sV[k * rk + s_sel[j]];
-    C[idx] = c;
+  {
+    double y[kRRItems];
+#pragma unroll
+    for (int t = 0; t < kRRItems; ++t) {
+      const int idx = tid + t * kRRThreads;
+      if (idx < rk * m) {
+        const int k = idx / m, j = idx - k * m;
+        y[t] = sV[k * rk + s_sel[j]];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kRRItems; ++t)
+      if (tid + t * kRRThreads < rk * m) sV[tid + t * kRRThreads] = y[t];
   }
+  for (int a = wave; a < ns; a += nwaves)
+    for (int k = lane; k < rk; k += 64) sA[a * rk + k] = Z[a * NS + k];
   __syncthreads();
+  lds_product<false>(ns, m, rk, sA, rk, sV, m, sV, m);
+  for (int idx = tid; idx < ns * m; idx += kRRThreads) C[idx] = sV[idx];
   // Gram blocks of the next basis' X' = S C and P' = S C0 (C0: the rows of X zeroed), for the
-  // iterations that sum only the new W's columns: T = G C, T0 = G C0 (into T1), then
-  // Gp = [C C0]^T [T T0] (upper triangle used), for G_K and G_M
+  // iterations that sum only the new W's columns: T = G C, T0 = G C0, then Gp = [C C0]^T [T T0] (upper
+  // triangle used), for G_K and G_M.  G in sA; C, T and T0 in sV (3 ns m values)
   const int m2 = 2 * m;
+  double *sC = sV, *sT = sV + ns * m, *sT0 = sT + ns * m;
   for (int mat = 0; mat < 2; ++mat) {
     const double* Gm = mat ? GM : GK;
-    for (int idx = tid; idx < ns * m; idx += blockDim.x) {
-      const int a = idx / m, j = idx % m;
-      double t = 0.0, t0 = 0.0;
-      for (int b = 0; b < ns; ++b) {
-        const double gab = 0.5 * (Gm[a * NS + b] + Gm[b * NS + a]) * C[b * m + j];
-        t += gab;
-        if (b >= m) t0 += gab;
-      }
-      T1[idx] = t;
-      T1[ns * m + idx] = t0;
-    }
     __syncthreads();
+    for (int a = wave; a < ns; a += nwaves)
+      for (int b = lane; b < ns; b += 64) sA[a * ns + b] = 0.5 * (Gm[a * NS + b] + Gm[b * NS + a]);
+    __syncthreads();
+    lds_product<false>(ns, m, ns, sA, ns, sC, m, sT, m);
+    lds_product<false>(ns, m, ns - m, sA + m, ns, sC + m * m, m, sT0, m);
     double* out = Gp + ((int64_t)v * 2 + mat) * m2 * m2;
     for (int idx = tid; idx < m2 * m2; idx += blockDim.x) {
-      const int i = idx / m2, j = idx % m2;
+      const int i = idx / m2, j = idx - i * m2;
       if (j < i) continue;
-      const double* Tj = T1 + (j < m ? 0 : ns * m);
+      const double* Tj = j < m ? sT : sT0;
       const int jc = j < m ? j : j - m, ic = i < m ? i : i - m;
       double g = 0.0;
-      for (int a = (i < m ? 0 : m); a < ns; ++a) g += C[a * m + ic] * Tj[a * m + jc];
+#pragma unroll 8
+      for (int a = (i < m ? 0 : m); a < ns; ++a) g += sC[a * m + ic] * Tj[a * m + jc];
       out[idx] = g;
     }
-    __syncthreads();
   }
 }
 
@@ -1276,7 +1417,6 @@ struct LobWork {
   double* G;
   double* C;
   double* Z;
-  double* T1;
   double* Gp;  // [nvar][2][2m][2m] Gram blocks of the next X and P (upper triangles)
   double* rc;  // two-level: [nvar][ld][m] restricted residuals and coarse solutions
   double* zc;
@@ -1323,7 +1463,6 @@ LobWork layout_lob(char* base, const LobParams& p, int64_t ld = 0) {
   w.G = (double*)take(nv * 2 * NS * NS * (int64_t)sizeof(double));
   w.C = (double*)take(nv * NS * p.m * (int64_t)sizeof(double));
   w.Z = (double*)take(nv * NS * NS * (int64_t)sizeof(double));
-  w.T1 = (double*)take(nv * NS * NS * (int64_t)sizeof(double));
   w.Gp = (double*)take(nv * 2 * 4 * (int64_t)p.m * p.m * (int64_t)sizeof(double));
   if (ld > 0) {
     w.rc = (double*)take(nv * ld * p.m * (int64_t)sizeof(double));
@@ -1371,10 +1510,11 @@ void launch_lob_coarse(hipStream_t st, const LobParams& p, const LobCoarse& cc, 
 template <int D, int LAYOUT>
 int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
                const uint8_t* fixed, double* X, double* lam, double* res, int32_t* iters,
-               int32_t* vstatus, const LobWork& w, const LobParams& p, const fe_lobpcg_opts* o,
+               int32_t* vstatus, const LobWork& w, LobParams p, const fe_lobpcg_opts* o,
                fe_lobpcg_stats* stats, const LobCoarse& cc) {
   hipStream_t st = h->stream;
   const int nv = p.nvar;
+  if (cc.C) p.nchunk_r = (int)std::min<int64_t>(p.nchunk_r, cc.C->n_agg);  // no chunk without an aggregate
   if (cc.C) FE_CHECK_HIP(hipMemsetAsync(w.rc, 0, (size_t)nv * cc.ld * p.m * sizeof(double), st));
   const dim3 gvar((unsigned)ceil_div(nv, 64));
   hipLaunchKernelGGL(k_lob_init, gvar, dim3(64), 0, st, p, w.st);
@@ -1404,7 +1544,7 @@ int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
   const dim3 gres((unsigned)p.nchunk_r, nv);
   const dim3 ggram((unsigned)p.nchunk_g, nv);
   const int NS = 3 * p.m;
-  const dim3 ggsum((unsigned)ceil_div(2 * NS * NS, kThreads), nv);
+  const dim3 ggsum((unsigned)ceil_div(2 * NS * NS, kSumEntries), nv);
   const size_t rr_lds = 2 * (size_t)NS * NS * sizeof(double);
   FE_CHECK_HIP(hipFuncSetAttribute((const void*)k_lob_rr, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)rr_lds));
@@ -1419,7 +1559,7 @@ int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
       hipLaunchKernelGGL(k_lob_gsum_w, ggsum, dim3(kThreads), 0, st, p, w.st, w.gpart, w.Gp, w.G);
     }
     hipLaunchKernelGGL(k_lob_rr, dim3(nv), dim3(kRRThreads), rr_lds, st, p, w.st, w.rpart, w.G, w.Z,
-                       w.T1, w.C, w.Gp);
+                       w.C, w.Gp);
     launch_update(st, p, w.st, w.blk, w.C);
     hipLaunchKernelGGL(k_lob_flip, gvar, dim3(64), 0, st, p, w.st);
     FE_CHECK_LAUNCH();
@@ -1446,8 +1586,12 @@ int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
       }
       constexpr int NC = D == 3 ? 6 : D == 2 ? 3 : 1;
       if (cc.C) {
-        hipLaunchKernelGGL((k_lob_resid_agg<D, NC>), gres, dim3(kThreads), 0, st, p, *cc.C, cc.ld, T,
-                           o->t_stride, fixed, w.st, w.blk, w.rpart, w.rc);
+        // an aggregate is one workgroup's: 1,024 threads where they all find a node of an average one (20^3
+        // cubes, 4 variants, 12 columns: 182 us with 256 threads, 78 with 1,024)
+        auto resid = p.nb / cc.C->n_agg >= 1024 / p.m ? k_lob_resid_agg<D, NC, 1024> : k_lob_resid_agg<D, NC, kThreads>;
+        const int nt = p.nb / cc.C->n_agg >= 1024 / p.m ? 1024 : kThreads;
+        hipLaunchKernelGGL(resid, gres, dim3(nt), 0, st, p, *cc.C, cc.ld, T, o->t_stride, fixed, w.st, w.blk,
+                           w.rpart, w.rc);
         launch_lob_coarse<D, NC>(st, p, cc, w);
       } else {
         hipLaunchKernelGGL((k_lob_resid<D>), gres, dim3(kThreads), 0, st, p, T, o->t_stride, fixed,

@@ -240,247 +240,309 @@ __global__ void k_identity_pad(int64_t n, int64_t ld, double* __restrict__ A) {
 // ---------------------------------------------------------------------------------------------------
 // blocked Gauss-Jordan inversion (in place, FP64)
 // ---------------------------------------------------------------------------------------------------
-// C (64 x 64, global) = alpha * X * Y (+ C if accumulate), X and Y 64 x 64 tiles in LDS.
-__device__ void tile_gemm_store(double (*sX)[kNB + 1], double (*sY)[kNB + 1], double* __restrict__ Cg,
-                                int64_t ld, double alpha, bool accumulate) {
-  // 256 threads, 4 x 4 outputs each
-  const int tr = (threadIdx.x / 16) * 4, tc = (threadIdx.x % 16) * 4;
-  double acc[4][4] = {};
-  for (int kk = 0; kk < kNB; ++kk) {
-    double x[4], y[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      x[a] = sX[tr + a][kk];
-      y[a] = sY[kk][tc + a];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] += x[a] * y[b];
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      double* c = Cg + (int64_t)(tr + a) * ld + tc + b;
-      *c = (accumulate ? *c : 0.0) + alpha * acc[a][b];
-    }
+typedef double gj_d4 __attribute__((ext_vector_type(4)));
+
+// 1 / x: the hardware's estimate and two Newton steps.
+__device__ inline double gj_recip(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = y + y * (1.0 - x * y);
+  return y + y * (1.0 - x * y);
 }
 
-// acc = X * Y for the 4 x 4 outputs (rows tr.., columns tc..) of this thread, 256 threads.
-__device__ inline void tile_gemm_acc(double (*sX)[kNB + 1], double (*sY)[kNB + 1], double (&acc)[4][4]) {
-  const int tr = (threadIdx.x / 16) * 4, tc = (threadIdx.x % 16) * 4;
+template <int P>
+__device__ inline void gj16_step(gj_d4& a, int lane) {
+  constexpr int q = P >> 2, g = P & 3;  // the pivot row's register and lane group
+  const int c = lane & 15;
+  const long long bits = __double_as_longlong(a[q]);
+  const double piv = __longlong_as_double(
+      ((long long)__builtin_amdgcn_readlane((int)(bits >> 32), g * 16 + P) << 32) |
+      (unsigned)__builtin_amdgcn_readlane((int)bits, g * 16 + P));
+  const double row = __shfl(a[q], g * 16 + c, 64);
+  gj_d4 col;
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int i = 0; i < 4; ++i) col[i] = dpp_move<0x150 | P>(a[i]);  // lane P of every row of 16
+  const double prow = (c == P ? 1.0 : row) * gj_recip(piv);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  for (int kk = 0; kk < kNB; ++kk) {
-    double x[4], y[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      x[a] = sX[tr + a][kk];
-      y[a] = sY[kk][tc + a];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] += x[a] * y[b];
-  }
+  for (int i = 0; i < 4; ++i) a[i] = (c == P ? 0.0 : a[i]) - col[i] * prow;
+  if ((lane >> 4) == g) a[q] = prow;
 }
 
-constexpr int kGjThreads = 256;
+// In-place inverse of a 16 x 16 SPD block by one wavefront, no pivoting, held as the matrix cores leave a
+// product: lane l has column l % 16 of rows 4 i + l / 16.
+__device__ inline void gj16(gj_d4& a) {
+  const int lane = threadIdx.x & 63;
+  gj16_step<0>(a, lane), gj16_step<1>(a, lane), gj16_step<2>(a, lane), gj16_step<3>(a, lane);
+  gj16_step<4>(a, lane), gj16_step<5>(a, lane), gj16_step<6>(a, lane), gj16_step<7>(a, lane);
+  gj16_step<8>(a, lane), gj16_step<9>(a, lane), gj16_step<10>(a, lane), gj16_step<11>(a, lane);
+  gj16_step<12>(a, lane), gj16_step<13>(a, lane), gj16_step<14>(a, lane), gj16_step<15>(a, lane);
+}
 
-// A 64 x 64 tile into LDS by the 256 threads: each thread's eight 16-byte loads are issued together
-// (the rows are 16-byte aligned: ld and the tile offsets are multiples of 64).
-__device__ void load_tile(const double* __restrict__ A, int64_t ld, int bi, int bj,
-                          double (*s)[kNB + 1]) {
+// In-place inverse of an SPD matrix of nblk x nblk blocks of 16 x 16 in LDS (row-major, leading dimension
+// lda) by NW >= nblk wavefronts: Gauss-Jordan by block rows, the block products on the matrix cores.
+// Bound by the chain of pivots (one element after the other), so a pivot block is inverted in one wavefront's
+// registers, without barriers, as soon as its own update is done and while the other wavefronts do theirs;
+// two barriers per 16 pivots.  (One barrier and one division per pivot took about 30 us for 64 x 64.)
+// The blocks of the column of block p are those of its row transposed (negated where exactly one
+// of the two has been eliminated), so only the row is read.  sR: 16 rows of leading dimension ldr >= 16 nblk.
+template <int NW>
+__device__ void gj_invert_lds(double* s, int lda, int nblk, double* sR, int ldr) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  auto at = [&](int bi, int bj) { return s + bi * 16 * lda + bj * 16; };
+  auto load = [&](const double* b, gj_d4& v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = b[(4 * i + g) * lda + c];
+  };
+  auto store = [&](double* b, const gj_d4& v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[(4 * i + g) * lda + c] = v[i];
+  };
+  gj_d4 R = {0.0, 0.0, 0.0, 0.0};  // this wavefront's block of the pivot row
+  if (wave == 0) {
+    gj_d4 v;
+    load(at(0, 0), v);
+    gj16(v);
+    store(at(0, 0), v);
+  }
+  __syncthreads();
+  for (int p = 0; p < nblk; ++p) {
+    // the pivot row: R_pj = A_pp^-1 A_pj by wavefront j; the previous one, read until here, into its place
+    if (wave < nblk) {
+      if (p > 0 && wave != p - 1) store(at(p - 1, wave), R);
+      if (wave != p) {
+        R = gj_d4{0.0, 0.0, 0.0, 0.0};
+        const double *d = at(p, p), *a = at(p, wave);
+#pragma unroll
+        for (int k = 0; k < 16; k += 4)
+          R = __builtin_amdgcn_mfma_f64_16x16x4f64(d[c * lda + k + g], a[(k + g) * lda + c], R, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sR[(4 * i + g) * ldr + wave * 16 + c] = R[i];
+      }
+    }
+    __syncthreads();
+    // A_ij -= A_ip R_pj with A_ip = +-A_pi^T
+    auto update = [&](int i, int j, gj_d4& v) {
+      const double sgn = i < p ? 1.0 : -1.0;
+      const double *a = at(p, i), *r = sR + j * 16;
+      load(at(i, j), v);
+      gj_d4 ar = {0.0, 0.0, 0.0, 0.0};  // summed by itself: the small terms are rounded at their own size
+#pragma unroll
+      for (int k = 0; k < 16; k += 4)
+        ar = __builtin_amdgcn_mfma_f64_16x16x4f64(a[(k + g) * lda + c], r[(k + g) * ldr + c], ar, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] += sgn * ar[q];
+    };
+    if (wave == 0 && p + 1 < nblk) {
+      gj_d4 v;
+      update(p + 1, p + 1, v);
+      gj16(v);
+      store(at(p + 1, p + 1), v);
+    } else if (wave > 0) {
+      for (int t = wave - 1; t < (nblk - 1) * (nblk - 1); t += NW - 1) {
+        int i = t / (nblk - 1), j = t % (nblk - 1);
+        i += i >= p;
+        j += j >= p;
+        if (i == p + 1 && j == p + 1) continue;
+        gj_d4 v;
+        update(i, j, v);
+        store(at(i, j), v);
+      }
+    }
+    // A_ip = -A_ip A_pp^-1, the transposed row
+    if (wave < nblk && wave != p) {
+      const double sgn = wave < p ? 1.0 : -1.0;
+      double* b = at(wave, p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[c * lda + 4 * i + g] = sgn * R[i];
+    }
+    __syncthreads();
+  }
+  if (wave < nblk - 1) store(at(nblk - 1, wave), R);
+  __syncthreads();
+}
+
+constexpr int kGjThreads = 256, kGjLd = kNB + 1;
+
+// A 64 x 64 tile into LDS by the 256 threads, times sgn: each thread's eight 16-byte loads are issued
+// together (the rows are 16-byte aligned: ld and the tile offsets are multiples of 64).
+__device__ void load_tile(const double* __restrict__ A, int64_t ld, double sgn, double* __restrict__ s) {
   constexpr int kPer = kNB * kNB / 2 / kGjThreads;
   double2 v[kPer];
 #pragma unroll
   for (int it = 0; it < kPer; ++it) {
     const int idx = 2 * ((int)threadIdx.x + it * kGjThreads);
-    const int r = idx / kNB, c = idx % kNB;
-    v[it] = *reinterpret_cast<const double2*>(A + (int64_t)(bi * kNB + r) * ld + bj * kNB + c);
+    v[it] = *reinterpret_cast<const double2*>(A + (int64_t)(idx / kNB) * ld + idx % kNB);
   }
 #pragma unroll
   for (int it = 0; it < kPer; ++it) {
     const int idx = 2 * ((int)threadIdx.x + it * kGjThreads);
-    const int r = idx / kNB, c = idx % kNB;
-    s[r][c] = v[it].x;
-    s[r][c + 1] = v[it].y;
+    double* d = s + idx / kNB * kGjLd + idx % kNB;
+    d[0] = sgn * v[it].x;
+    d[1] = sgn * v[it].y;
   }
 }
 
-// In-place Gauss-Jordan inversion of a 64 x 64 tile by 256 threads: thread (g, c) keeps rows
-// 16g..16g+15 of column c in a[].  Each elimination step broadcasts the pivot row, the pivot column and
-// the pivot's reciprocal (formed once, by the pivot's owner) through LDS buffers that alternate
-// between steps, so one barrier per step separates their writes from the reads.  No pivoting: the
-// diagonal blocks met by the blocked elimination of an SPD matrix are SPD.
-struct GjLds {
-  double row[2][kNB], col[2][kNB], piv[2];
-};
+// A wavefront's 32 x 32 quadrant of a 64 x 64 tile as four 16 x 16 accumulators; f(value, row, column).
+template <typename F>
+__device__ __forceinline__ void each_of_tile(gj_d4 (&acc)[2][2], F f) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        double v = acc[x][y][i];
+        f(v, (wave >> 1) * 32 + x * 16 + 4 * i + (lane >> 4), (wave & 1) * 32 + y * 16 + (lane & 15));
+        acc[x][y][i] = v;
+      }
+}
 
-__device__ void gj_invert_tile(double (&a)[16], GjLds& L) {
-  const int c = threadIdx.x % kNB, g = threadIdx.x / kNB;
-  for (int pb = 0; pb < kNB / 16; ++pb) {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int p = pb * 16 + q, buf = q & 1;
-      if (g == pb) {
-        L.row[buf][c] = a[q];
-        if (c == p) L.piv[buf] = 1.0 / a[q];
-      }
-      if (c == p)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) L.col[buf][g * 16 + i] = a[i];
-      __syncthreads();
-      const double prow = (c == p ? 1.0 : L.row[buf][c]) * L.piv[buf];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = g * 16 + i;
-        a[i] = (r == p) ? prow : (c == p ? 0.0 : a[i]) - L.col[buf][r] * prow;
-      }
-    }
+// acc += X Y of two 64 x 64 tiles in LDS.
+__device__ __forceinline__ void tile_product(const double* sX, const double* sY, gj_d4 (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const double* a = sX + ((wave >> 1) * 32 + c) * kGjLd + g;
+  const double* b = sY + g * kGjLd + (wave & 1) * 32 + c;
+#pragma unroll 4
+  for (int k = 0; k < kNB; k += 4) {
+    const double a0 = a[k], a1 = a[16 * kGjLd + k], b0 = b[k * kGjLd], b1 = b[k * kGjLd + 16];
+    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
+    acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
+    acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
+    acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
   }
 }
 
-// S = inv(A_00) (the first pivot block; later ones are inverted inside k_gj_update).
+// S = inv(tile in sX), all threads.
+__device__ void invert_pivot(double* sX, double* sR, double* __restrict__ S) {
+  gj_invert_lds<kGjThreads / 64>(sX, kGjLd, kNB / 16, sR, kNB);
+  for (int idx = threadIdx.x; idx < kNB * kNB; idx += kGjThreads) S[idx] = sX[idx / kNB * kGjLd + idx % kNB];
+}
+
+// S = inv(A_00) (the first pivot block; later ones are inverted inside k_gj_step).
 __global__ __launch_bounds__(kGjThreads) void k_gj_inv(int64_t ld, const double* __restrict__ A,
                                                        double* __restrict__ S) {
-  __shared__ GjLds L;
-  const int c = threadIdx.x % kNB, g = threadIdx.x / kNB;
-  double a[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) a[i] = A[(int64_t)(g * 16 + i) * ld + c];
-  gj_invert_tile(a, L);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) S[(g * 16 + i) * kNB + c] = a[i];
-}
-
-// Step k of the blocked elimination reads A (the matrix after step k-1) and writes B; S = inv(A_kk).
-// Part 1 (workgroup per block column j): B_kj = S A_kj, B_kk = S.
-__global__ __launch_bounds__(kGjThreads) void k_gj_row(int64_t ld, int k, const double* __restrict__ A,
-                                                       double* __restrict__ B,
-                                                       const double* __restrict__ S) {
-  __shared__ double sP[kNB][kNB + 1], sT[kNB][kNB + 1];
-  const int j = blockIdx.x;
-  if (j == k) {
-    for (int idx = threadIdx.x; idx < kNB * kNB; idx += blockDim.x)
-      B[(int64_t)(k * kNB + idx / kNB) * ld + k * kNB + idx % kNB] = S[idx];
-    return;
-  }
-  for (int idx = threadIdx.x; idx < kNB * kNB; idx += blockDim.x) sP[idx / kNB][idx % kNB] = S[idx];
-  load_tile(A, ld, k, j, sT);
+  __shared__ double sX[kNB * kGjLd], sR[16 * kNB];
+  load_tile(A, ld, 1.0, sX);
   __syncthreads();
-  tile_gemm_store(sP, sT, B + (int64_t)(k * kNB) * ld + j * kNB, ld, 1.0, false);
+  invert_pivot(sX, sR, S);
 }
 
-// Part 2 (workgroup per block (i, j), i != k): B_ij = A_ij - A_ik B_kj (j != k), B_ik = -A_ik S.
-// The workgroup of block (k+1, k+1) then inverts its new block into Snext, the next step's S.
-__global__ __launch_bounds__(kGjThreads) void k_gj_update(int64_t ld, int k, const double* __restrict__ A,
-                                                          double* __restrict__ B,
-                                                          const double* __restrict__ S,
-                                                          double* __restrict__ Snext) {
-  __shared__ double sX[kNB][kNB + 1], sY[kNB][kNB + 1];
-  __shared__ GjLds L;
+// Step k of the blocked elimination reads A (the matrix after step k-1) and writes B; S = inv(A_kk):
+// B_kk = S, B_kj = S A_kj, B_ij = A_ij - A_ik S A_kj, B_ik = -A_ik S.  A workgroup takes block column j of
+// `rows` block rows and forms S A_kj for itself (one launch per step; `rows` so that about one workgroup
+// per CU shares it).  Workgroup 0 does block (k+1, k+1) alone and then inverts it into Snext, the next
+// step's S: its load, two products and inversion are the step's critical path.  1,280 x 1,280: 22.7 us a step,
+// where a launch for the block row and one for the rest took 58.
+__global__ __launch_bounds__(kGjThreads) void k_gj_step(int64_t ld, int k, int rows, const double* __restrict__ A,
+                                                        double* __restrict__ B, const double* __restrict__ S,
+                                                        double* __restrict__ Snext) {
+  __shared__ double sX[kNB * kGjLd], sY[kNB * kGjLd], sR[16 * kNB];
   const int nb = (int)(ld / kNB);
-  const int i = blockIdx.x / nb, j = blockIdx.x % nb;
-  if (i == k) return;
-  load_tile(A, ld, i, k, sX);
+  const bool pivot = blockIdx.x == 0;
+  if (pivot && k + 1 == nb) return;
+  const int t = (int)blockIdx.x - 1;
+  const int j = pivot ? k + 1 : t % nb;
+  const int i0 = pivot ? k + 1 : t / nb * rows, i1 = pivot ? k + 2 : min(i0 + rows, nb);
+  auto tile = [&](auto* M, int bi, int bj) { return M + (int64_t)bi * kNB * ld + bj * kNB; };
+  gj_d4 acc[2][2] = {};
   if (j == k) {
-    for (int idx = threadIdx.x; idx < kNB * kNB; idx += blockDim.x) sY[idx / kNB][idx % kNB] = S[idx];
-    __syncthreads();
-    tile_gemm_store(sX, sY, B + (int64_t)(i * kNB) * ld + k * kNB, ld, -1.0, false);
-    return;
-  }
-  load_tile(B, ld, k, j, sY);
-  // this thread's 4 x 4 outputs of A_ij, loaded before the product so that their latency overlaps it
-  const int tr = (threadIdx.x / 16) * 4, tc = (threadIdx.x % 16) * 4;
-  double aij[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const double* row = A + (int64_t)(i * kNB + tr + a) * ld + j * kNB + tc;
-    const double2 lo = *reinterpret_cast<const double2*>(row);
-    const double2 hi = *reinterpret_cast<const double2*>(row + 2);
-    aij[a][0] = lo.x, aij[a][1] = lo.y, aij[a][2] = hi.x, aij[a][3] = hi.y;
-  }
-  __syncthreads();
-  double acc[4][4];
-  tile_gemm_acc(sX, sY, acc);
-  const bool pivot_next = (i == k + 1 && j == k + 1);
-  if (pivot_next) __syncthreads();  // sX is reused for the new block below
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    double v[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      v[b] = aij[a][b] - acc[a][b];
-      if (pivot_next) sX[tr + a][tc + b] = v[b];
+    load_tile(S, kNB, -1.0, sY);
+    if (i0 == 0) {
+      double* out = tile(B, k, k);
+      for (int idx = threadIdx.x; idx < kNB * kNB; idx += kGjThreads)
+        out[(int64_t)(idx / kNB) * ld + idx % kNB] = S[idx];
     }
-    double* row = B + (int64_t)(i * kNB + tr + a) * ld + j * kNB + tc;
-    *reinterpret_cast<double2*>(row) = double2{v[0], v[1]};
-    *reinterpret_cast<double2*>(row + 2) = double2{v[2], v[3]};
+  } else {
+    load_tile(S, kNB, 1.0, sX);
+    load_tile(tile(A, k, j), ld, 1.0, sY);
+    __syncthreads();
+    tile_product(sX, sY, acc);
+    __syncthreads();
+    double* out = tile(B, k, j);
+    const bool keep = !pivot && i0 == 0;
+    each_of_tile(acc, [&](double& v, int r, int c) {
+      sY[r * kGjLd + c] = -v;
+      if (keep) out[(int64_t)r * ld + c] = v;
+    });
   }
-  if (!pivot_next) return;
-  // the next pivot block (this workgroup's own output): invert it into Snext
+  for (int i = i0; i < i1; ++i) {
+    if (i == k || (!pivot && i == k + 1 && j == k + 1)) continue;
+    // A_ij is loaded before the product so that its latency overlaps it, and added after it: the
+    // product's terms are rounded at their own size
+    const double* aij = tile(A, i, j);
+    gj_d4 old[2][2];
+    each_of_tile(old, [&](double& v, int r, int c) { v = j == k ? 0.0 : aij[(int64_t)r * ld + c]; });
+    each_of_tile(acc, [&](double& v, int, int) { v = 0.0; });
+    load_tile(tile(A, i, k), ld, 1.0, sX);
+    __syncthreads();
+    tile_product(sX, sY, acc);
+    __syncthreads();
+    double* out = tile(B, i, j);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) acc[x][y] += old[x][y];
+    each_of_tile(acc, [&](double& v, int r, int c) {
+      out[(int64_t)r * ld + c] = v;
+      if (pivot) sX[r * kGjLd + c] = v;
+    });
+  }
+  if (!pivot) return;
   __syncthreads();
-  const int c = threadIdx.x % kNB, g = threadIdx.x / kNB;
-  double t[16];
-#pragma unroll
-  for (int q = 0; q < 16; ++q) t[q] = sX[g * 16 + q][c];
-  gj_invert_tile(t, L);
-#pragma unroll
-  for (int q = 0; q < 16; ++q) Snext[(g * 16 + q) * kNB + c] = t[q];
+  invert_pivot(sX, sR, Snext);
 }
 
-// Block-diagonal space: one workgroup per segment inverts its block (n_s <= 128, SPD, no pivoting) by
-// in-place Gauss-Jordan in LDS, then writes the symmetrised inverse and its FP32 copy.
+// Block-diagonal space: one workgroup per segment inverts its block (n_s <= 128, SPD, no pivoting) in
+// LDS, padded with the identity to whole 16 x 16 blocks, then writes the symmetrised inverse and its FP32 copy.
 constexpr int kSegMax = 128;
 constexpr int kSegThreads = 1024;
 
+__host__ __device__ inline int seg_pad(int n) { return (n + 15) / 16 * 16; }
+__host__ __device__ inline size_t seg_lds(int n) {  // the padded block, odd leading dimension, and the pivot row
+  return (size_t)(seg_pad(n) * (seg_pad(n) + 1) + 16 * seg_pad(n)) * sizeof(double);
+}
+
 __global__ __launch_bounds__(kSegThreads) void k_coarse_inv_seg(fe_coarse C, double* __restrict__ A,
                                                                float* __restrict__ A32) {
-  extern __shared__ double sA[];  // [n][n]
-  __shared__ double s_row[kSegMax], s_col[kSegMax];
+  extern __shared__ double sA[];  // [np][np + 1], then the pivot row
   const int sg = blockIdx.x;
   const int n = C.nc * (C.agg_seg[sg + 1] - C.agg_seg[sg]);
   if (n == 0) return;
+  const int np = seg_pad(n), lda = np + 1;
   double* Ag = A + C.blk_ofs[sg];
-  for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) sA[idx] = Ag[idx];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i = wave; i < np; i += kSegThreads / 64)
+    for (int j = lane; j < np; j += 64) sA[i * lda + j] = i < n && j < n ? Ag[i * n + j] : (i == j ? 1.0 : 0.0);
   __syncthreads();
-  for (int p = 0; p < n; ++p) {
-    const double piv = 1.0 / sA[p * n + p];
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      s_row[j] = (j == p ? 1.0 : sA[p * n + j]) * piv;
-      s_col[j] = sA[j * n + p];
+  gj_invert_lds<kSegThreads / 64>(sA, lda, np / 16, sA + np * lda, np);
+  for (int i = wave; i < n; i += kSegThreads / 64)
+    for (int j = lane; j < n; j += 64) {
+      const double v = 0.5 * (sA[i * lda + j] + sA[j * lda + i]);
+      Ag[i * n + j] = v;
+      if (A32) A32[C.blk_ofs[sg] + i * n + j] = (float)v;
     }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) {
-      const int i = idx / n, j = idx - i * n;
-      sA[idx] = (i == p) ? s_row[j] : (j == p ? 0.0 : sA[idx]) - s_col[i] * s_row[j];
-    }
-    __syncthreads();
-  }
-  for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) {
-    const int i = idx / n, j = idx - i * n;
-    const double v = 0.5 * (sA[idx] + sA[j * n + i]);
-    Ag[idx] = v;
-    if (A32) A32[C.blk_ofs[sg] + idx] = (float)v;
-  }
 }
 
-// Symmetrise the inverse (average with its transpose) and make the FP32 copy.
-__global__ void k_sym_cast(int64_t n, int64_t ld, double* __restrict__ A, float* __restrict__ A32) {
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= n * n) return;
-  const int64_t r = t / n, c = t % n;
-  if (r > c) return;
-  const double v = 0.5 * (A[r * ld + c] + A[c * ld + r]);
-  A[r * ld + c] = v;
-  A[c * ld + r] = v;
-  if (A32) {
-    A32[r * ld + c] = (float)v;
-    A32[c * ld + r] = (float)v;
+// The inverse (in src, which may be A) symmetrised into A (average with its transpose) with its FP32 copy.  A
+// workgroup takes a 32 x 32 tile and its mirror image, through LDS so that both are read and written by rows (1,280 x 1,280: 25 us without, 7 with).
+constexpr int kSymTile = 32;
+__global__ __launch_bounds__(256) void k_sym_cast(int64_t n, int64_t ld, const double* src, double* A,
+                                                  float* __restrict__ A32) {
+  __shared__ double s[2][kSymTile][kSymTile + 1];
+  if (blockIdx.y > blockIdx.x) return;
+  const int64_t r0 = (int64_t)blockIdx.y * kSymTile, c0 = (int64_t)blockIdx.x * kSymTile;
+  const int c = threadIdx.x % kSymTile;
+  for (int r = threadIdx.x / kSymTile; r < kSymTile; r += 256 / kSymTile) {
+    s[0][r][c] = src[(r0 + r) * ld + c0 + c];
+    s[1][r][c] = src[(c0 + r) * ld + r0 + c];
+  }
+  __syncthreads();
+  for (int r = threadIdx.x / kSymTile; r < kSymTile; r += 256 / kSymTile) {
+    const double u = 0.5 * (s[0][r][c] + s[1][c][r]), v = 0.5 * (s[1][r][c] + s[0][c][r]);
+    A[(r0 + r) * ld + c0 + c] = u;
+    A[(c0 + r) * ld + r0 + c] = v;
+    if (A32 && r0 + r < n && c0 + c < n) A32[(r0 + r) * ld + c0 + c] = (float)u;
+    if (A32 && c0 + r < n && r0 + c < n) A32[(c0 + r) * ld + r0 + c] = (float)v;
   }
 }
 
@@ -908,7 +970,7 @@ extern "C" int fe_coarse_operator(fe_handle* h, const fe_bsr* A, const fe_coarse
     // block-diagonal: one workgroup per segment inverts its block in LDS
     FE_CHECK_LAUNCH();
     if (!invert) return FE_OK;
-    const size_t lds = (size_t)C->max_block * C->max_block * sizeof(double);
+    const size_t lds = seg_lds(C->max_block);
     if (lds > 64 * 1024)
       FE_CHECK_HIP(hipFuncSetAttribute((const void*)k_coarse_inv_seg,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -929,16 +991,15 @@ extern "C" int fe_coarse_operator(fe_handle* h, const fe_bsr* A, const fe_coarse
   double* cur = Ac;
   double* nxt = scratch;
   hipLaunchKernelGGL(k_gj_inv, dim3(1), dim3(kGjThreads), 0, st, ld, Ac, Sb[0]);
+  const int rows = (nb * nb + 255) / 256;
+  const unsigned wgs = 1 + (unsigned)(nb * ceil_div(nb, rows));
   for (int k = 0; k < nb; ++k) {
-    hipLaunchKernelGGL(k_gj_row, dim3((unsigned)nb), dim3(kGjThreads), 0, st, ld, k, cur, nxt, Sb[k & 1]);
-    hipLaunchKernelGGL(k_gj_update, dim3((unsigned)(nb * nb)), dim3(kGjThreads), 0, st, ld, k, cur, nxt,
-                       Sb[k & 1], Sb[(k + 1) & 1]);
+    hipLaunchKernelGGL(k_gj_step, dim3(wgs), dim3(kGjThreads), 0, st, ld, k, rows, cur, nxt, Sb[k & 1],
+                       Sb[(k + 1) & 1]);
     std::swap(cur, nxt);
   }
-  if (cur != Ac) FE_CHECK_HIP(hipMemcpyAsync(Ac, cur, (size_t)ld * ld * sizeof(double),
-                                             hipMemcpyDeviceToDevice, st));
-  hipLaunchKernelGGL(k_sym_cast, dim3((unsigned)ceil_div(nct * nct, 256)), dim3(256), 0, st, nct, ld,
-                     Ac, Ac32);
+  const unsigned nt = (unsigned)(ld / kSymTile);
+  hipLaunchKernelGGL(k_sym_cast, dim3(nt, nt), dim3(256), 0, st, nct, ld, cur, Ac, Ac32);
   FE_CHECK_LAUNCH();
   return FE_OK;
 }

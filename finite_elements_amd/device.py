@@ -79,6 +79,30 @@ class Context:
             t = t.to(dtype)
         return t.to(self.torch_device)
 
+    #: arrays up to this size share one copy to the device: a copy costs the host about 17 us whatever its
+    #: size, and collecting 64 KiB about 5
+    PACK_BYTES = 64 * 1024
+
+    def tensors(self, *arrays):
+        """``tensor`` of each array (None stays None), the small ones in one copy."""
+        arrays = [None if a is None else np.ascontiguousarray(a) for a in arrays]
+        small = [k for k, a in enumerate(arrays) if a is not None and 0 < a.nbytes <= self.PACK_BYTES]
+        out = [None if a is None or k in small else self.tensor(a) for k, a in enumerate(arrays)]
+        ends = np.cumsum([-(-arrays[k].nbytes // 512) * 512 for k in small])  # aligned as allocations are
+        if small:
+            host = np.empty(int(ends[-1]), dtype=np.uint8)
+            views = []
+            for k, end in zip(small, ends):
+                a = arrays[k]
+                off = int(end) - (-(-a.nbytes // 512) * 512)
+                host[off:off + a.nbytes] = a.reshape(-1).view(np.uint8)
+                views.append((k, off, a))
+            dev = self.tensor(host)
+            for k, off, a in views:
+                dtype = torch.as_tensor(a).dtype
+                out[k] = dev[off:off + a.nbytes].view(dtype).reshape(a.shape)
+        return out
+
     def empty(self, n, dtype=torch.float64):
         return torch.empty(int(n), dtype=dtype, device=self.torch_device)
 
@@ -190,10 +214,6 @@ class DeviceMesh:
         self.n_nodes = coords.shape[0]
         self.n_elem = conn.shape[0]
         self.plane_mode = plane_mode
-        self.x = ctx.tensor(coords[:, 0])
-        self.y = ctx.tensor(coords[:, 1])
-        self.z = ctx.tensor(coords[:, 2]) if coords.shape[1] > 2 else None
-        self.conn = ctx.tensor(np.ascontiguousarray(conn.T))
 
         def mat(key):
             v = materials.get(key)
@@ -202,15 +222,16 @@ class DeviceMesh:
             v = np.asarray(v, dtype=np.float64)
             if v.ndim == 0:
                 v = np.full(self.n_elem, float(v))
-            return ctx.tensor(v)
+            return v
 
         if kind == 'tri_elastic':
-            self.mat0, self.mat1, self.mat2 = mat('E'), mat('nu'), mat('thickness')
+            mats = mat('E'), mat('nu'), mat('thickness')
         elif kind == 'tet_elastic':
-            self.mat0, self.mat1, self.mat2 = mat('E'), mat('nu'), None
+            mats = mat('E'), mat('nu'), None
         else:
-            self.mat0, self.mat1, self.mat2 = mat('mu'), None, None
-        self.rho = mat('rho')
+            mats = mat('mu'), None, None
+        (self.x, self.y, self.z, self.conn, self.mat0, self.mat1, self.mat2, self.rho) = ctx.tensors(
+            coords[:, 0], coords[:, 1], coords[:, 2] if coords.shape[1] > 2 else None, conn.T, *mats, mat('rho'))
 
     def struct(self) -> _hip.FeMesh:
         return _hip.FeMesh(self.kind_id, self.plane_mode, self.n_elem, self.n_nodes, _vp(self.x),
@@ -245,17 +266,12 @@ class DeviceGraph:
         self.n_nodes = pat.n_nodes
         self.nnzb = pat.nnzb
         self.dof = pat.dof
-        self.bptr = ctx.tensor(pat.bptr)
-        self.bcol = ctx.tensor(pat.bcol)
-        self.inc_ptr = ctx.tensor(pat.inc_ptr)
-        self.inc = ctx.tensor(pat.inc)
-        self.bseg_ptr = ctx.tensor(pat.bseg_ptr)
-        self.bseg = ctx.tensor(pat.bseg.view(np.int16))
         rows = np.repeat(np.arange(self.n_nodes, dtype=np.int32), np.diff(pat.bptr))
         bdiag = np.full(max(self.n_nodes, 1), -1, dtype=np.int32)
         q = np.nonzero(pat.bcol == rows)[0]
         bdiag[rows[q]] = q
-        self.bdiag = ctx.tensor(bdiag)
+        (self.bptr, self.bcol, self.inc_ptr, self.inc, self.bseg_ptr, self.bseg, self.bdiag) = ctx.tensors(
+            pat.bptr, pat.bcol, pat.inc_ptr, pat.inc, pat.bseg_ptr, pat.bseg.view(np.int16), bdiag)
         self._conn = None
         self.set_schedule(pat.blk, pat.max_inc)
         self._padded = None
@@ -323,14 +339,10 @@ class DeviceGraph:
         wave-specialised persistent kernel with that many producer wavefronts."""
         blk = np.ascontiguousarray(np.asarray(blk, dtype=np.int32))
         wptr, welem, inc_sa, max_elem = element_schedule(self.pattern, blk)
-        self.blk = self.ctx.tensor(blk)
         self.n_blk = blk.size - 1
         self.max_inc = int(max_inc)
         self.threads = int(threads)
         self.max_elem = max_elem
-        self.welem_ptr = self.ctx.tensor(wptr)
-        self.welem = self.ctx.tensor(welem if welem.size else np.zeros(1, np.int32))
-        self.inc_sa = self.ctx.tensor((inc_sa if inc_sa.size else np.zeros(1, np.uint16)).view(np.int16))
         # per-workgroup header: every index the workgroup starts from, in one 48-byte record
         p = self.pattern
         n0, n1 = blk[:-1].astype(np.int64), blk[1:].astype(np.int64)
@@ -342,7 +354,10 @@ class DeviceGraph:
             hdr[:, 4], hdr[:, 5] = p.inc_ptr[n0], p.inc_ptr[n1] - p.inc_ptr[n0]
             hdr[:, 6], hdr[:, 7] = B0, B1 - B0
             hdr[:, 8], hdr[:, 9] = p.bseg_ptr[B0], p.bseg_ptr[B1] - p.bseg_ptr[B0]
-        self.wg_hdr = self.ctx.tensor(hdr.reshape(-1) if hdr.size else np.zeros(12, np.int32))
+        self.blk, self.welem_ptr, self.welem, self.inc_sa, self.wg_hdr = self.ctx.tensors(
+            blk, wptr, welem if welem.size else np.zeros(1, np.int32),
+            (inc_sa if inc_sa.size else np.zeros(1, np.uint16)).view(np.int16),
+            hdr.reshape(-1) if hdr.size else np.zeros(12, np.int32))
         self._hdr_host = hdr
         self._welem_ptr_host = wptr
         self._blk_host = blk
@@ -436,9 +451,7 @@ class PaddedGraph:
             pptr, bcol, src = pad_pattern(optr, ocol, a)
             src[src >= 0] = osrc[src[src >= 0]]
         self.nnzb = int(pptr[-1])
-        self.bptr = self.ctx.tensor(pptr)
-        self.bcol = self.ctx.tensor(bcol)
-        self.src_block = self.ctx.tensor(src)
+        self.bptr, self.bcol, self.src_block = self.ctx.tensors(pptr, bcol, src)
 
 
 def ordered_graph(graph, order: np.ndarray) -> PaddedGraph:
@@ -641,36 +654,23 @@ class DeviceCoarse:
     def __init__(self, ctx: Context, cs):
         self.ctx = ctx
         self.host = cs
-        t = ctx.tensor
-        self.node_agg = t(cs.node_agg)
-        self.agg_ptr = t(cs.agg_ptr)
-        self.agg_nodes = t(cs.agg_nodes)
-        self.pair_ptr = t(cs.pair_ptr)
-        self.pair_ij = t(np.ascontiguousarray(cs.pair_ij))
-        self.pair_q = t(cs.pair_q)
-        self.pair_row = t(cs.pair_row)
-        self.P = t(np.ascontiguousarray(cs.P.reshape(-1)))
-        self.P32 = _to_f32(ctx, self.P)
         xh = np.zeros((cs.P.shape[0], 3))
         xh[:, :cs.xhat.shape[1]] = cs.xhat
-        self.xhat = t(np.ascontiguousarray(xh.reshape(-1)))
+        seg = None, None, None
+        if cs.agg_seg is not None:
+            seg = cs.agg_seg, cs.seg_of_agg if cs.seg_of_agg.size else np.zeros(1, np.int32), cs.blk_ofs
+        (self.node_agg, self.agg_ptr, self.agg_nodes, self.pair_ptr, self.pair_ij, self.pair_q, self.pair_row,
+         self.P, self.xhat, self.fixed_bits, self.T, self.agg_seg, self.seg_of_agg, self.blk_ofs) = ctx.tensors(
+            cs.node_agg, cs.agg_ptr, cs.agg_nodes, cs.pair_ptr, cs.pair_ij, cs.pair_q, cs.pair_row,
+            cs.P.reshape(-1), xh.reshape(-1), cs.fixed_bits, cs.T.reshape(-1), *seg)
+        self.P32 = _to_f32(ctx, self.P)
         self.xhat32 = _to_f32(ctx, self.xhat)
-        self.fixed_bits = t(np.ascontiguousarray(cs.fixed_bits))
-        self.T = t(np.ascontiguousarray(cs.T.reshape(-1)))
         self.T32 = _to_f32(ctx, self.T)
         self.n_coarse = cs.n_coarse
         self.ld = int(_hip.load().fe_coarse_ld(cs.n_coarse))
         # block-diagonal space of a batch: one dense coarse block per mesh
-        if cs.agg_seg is not None:
-            self.n_seg = cs.agg_seg.size - 1
-            self.agg_seg = t(cs.agg_seg)
-            self.seg_of_agg = t(cs.seg_of_agg if cs.seg_of_agg.size else np.zeros(1, np.int32))
-            self.blk_ofs = t(cs.blk_ofs)
-            self.blk_total = int(cs.blk_ofs[-1])
-        else:
-            self.n_seg = 0
-            self.agg_seg = self.seg_of_agg = self.blk_ofs = None
-            self.blk_total = 0
+        self.n_seg = 0 if cs.agg_seg is None else cs.agg_seg.size - 1
+        self.blk_total = 0 if cs.agg_seg is None else int(cs.blk_ofs[-1])
 
     def struct(self) -> _hip.FeCoarse:
         cs = self.host

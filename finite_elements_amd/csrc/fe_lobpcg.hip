@@ -44,7 +44,8 @@ struct LobParams {
   int64_t nb, n, nnzb, nm;  // node rows, DOF rows, blocks, n*m
   int32_t m, n_wanted, largest, max_iter;
   double tol, drop;
-  int32_t nchunk_g, nchunk_r, nvar, pad;
+  int32_t nchunk_g, nchunk_r, nvar;
+  int32_t agg_parts;  // two-level: parts of an aggregate, each with its own partial of r_c
 };
 
 __device__ inline double* lob_block(double* base, const LobParams& p, int v, int idx) {
@@ -133,12 +134,12 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid(LobParams p, const doubl
 // constrained DOFs are zero, so W stays zero there.
 // --------------------------------------------------------------------------------------------------
 // K1 and K1b's restriction in one pass (two-level preconditioner): chunk b of the residual partials
-// takes aggregates [b n_agg / chunks, (b+1) n_agg / chunks) and walks their nodes (every node lies in
-// one aggregate), forming R, W = T R and the column norms as k_lob_resid does and r_c = P^T R (thread
+// takes aggregates [b n_agg / chunks, (b+1) n_agg / chunks), or part b % agg_parts of aggregate b / agg_parts,
+// and walks their nodes (every node lies in one aggregate), forming R, W = T R and the column norms as k_lob_resid does and r_c = P^T R (thread
 // (group g, column j) sums an aggregate's nodes g, g + npg, ..., then the groups are added in a
 // fixed order), so K X and M X are read once per iteration.
-template <int D, int NC, int NT>
-__global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, int64_t ld,
+template <int D, int NC>
+__global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coarse C, int64_t ld,
                                                             const double* __restrict__ T, int64_t t_stride,
                                                             const uint8_t* __restrict__ fixed,
                                                             const LobState* st, double* blk,
@@ -148,8 +149,8 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
   __shared__ int s_skip, s_cur;
   __shared__ double s_lam[kMaxBlock];
   __shared__ int s_lock[kMaxBlock];
-  __shared__ double s_rr[NT], s_bb[NT];
-  __shared__ double s_acc[NT][NC];
+  __shared__ double s_rr[kThreads], s_bb[kThreads];
+  __shared__ double s_acc[kThreads][NC];
   if (threadIdx.x == 0) {
     s_skip = st[v].done;
     s_cur = st[v].cur;
@@ -162,13 +163,15 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
   __syncthreads();
   if (s_skip) return;
   const int m = p.m;
-  const int npg = NT / m;
+  const int npg = kThreads / m;
   const int g = threadIdx.x / m, j = threadIdx.x % m;
   const double* KX = lob_block(blk, p, v, B_KX + s_cur);
   const double* MX = lob_block(blk, p, v, B_MX + s_cur);
   double* W = lob_block(blk, p, v, B_W);
   const double* Tv = T ? T + (int64_t)v * t_stride : nullptr;
-  const int64_t alo = C.n_agg * blockIdx.x / gridDim.x, ahi = C.n_agg * (blockIdx.x + 1) / gridDim.x;
+  const int parts = p.agg_parts, part = blockIdx.x % parts;  // parts > 1: n_agg * parts chunks
+  const int64_t chunk = blockIdx.x / parts, chunks = gridDim.x / parts;
+  const int64_t alo = C.n_agg * chunk / chunks, ahi = C.n_agg * (chunk + 1) / chunks;
   double* out = rpart + ((int64_t)v * gridDim.x + blockIdx.x) * 2 * m;
   const double lam = s_lam[j];
   double rr = 0.0, bb = 0.0;
@@ -177,8 +180,9 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[c] = 0.0;
     if (g < npg) {
-      const int32_t a0 = C.agg_ptr[agg], a1 = C.agg_ptr[agg + 1];
-      for (int32_t k = a0 + g; k < a1; k += npg) {
+      const int32_t a0 = C.agg_ptr[agg], na = C.agg_ptr[agg + 1] - a0;
+      const int32_t k1 = a0 + (int32_t)((int64_t)na * (part + 1) / parts);
+      for (int32_t k = a0 + (int32_t)((int64_t)na * part / parts) + g; k < k1; k += npg) {
         const int64_t i = C.agg_nodes[k];
         double R[D];
 #pragma unroll
@@ -209,7 +213,7 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
     for (int c = 0; c < NC; ++c) s_acc[threadIdx.x][c] = acc[c];
     __syncthreads();
     // the groups' sums over `ways` threads each (groups way, way + ways, ...), then those in order
-    const int outs = m * NC, ways = NT / outs, way = threadIdx.x / outs;
+    const int outs = m * NC, ways = kThreads / outs, way = threadIdx.x / outs;
     if (way < ways) {
       const int jj = threadIdx.x % m, c = threadIdx.x % outs / m;
       double sum = 0.0;
@@ -221,7 +225,7 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
     if (threadIdx.x < outs) {
       double sum = s_rr[threadIdx.x];
       for (int q = 1; q < ways; ++q) sum += s_rr[q * outs + threadIdx.x];
-      rc[((int64_t)v * ld + agg * NC + threadIdx.x / m) * m + threadIdx.x % m] = sum;
+      rc[(((int64_t)v * parts + part) * ld + agg * NC + threadIdx.x / m) * m + threadIdx.x % m] = sum;
     }
   }
   __syncthreads();
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(NT) void k_lob_resid_agg(LobParams p, fe_coarse C, 
   s_rr[threadIdx.x] = rr;
   s_bb[threadIdx.x] = bb;
   __syncthreads();
-  const int outs = 2 * m, ways = NT / outs, way = threadIdx.x / outs, x = threadIdx.x % outs;
+  const int outs = 2 * m, ways = kThreads / outs, way = threadIdx.x / outs, x = threadIdx.x % outs;
   if (way < ways) {
     const double* src = x < m ? s_rr + x : s_bb + x - m;
     double sum = 0.0;
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(kThreads) void k_lob_cgemm(LobParams p, int64_t ld,
   const int m = p.m;
   const int64_t r0 = (int64_t)blockIdx.x * kCgRows;
   const double* A = Ainv + (int64_t)v * ainv_stride;
-  const double* R = rc + (int64_t)v * ld * m;
+  const double* R = rc + (int64_t)v * p.agg_parts * ld * m;
   constexpr int kPer = (kCgRows * kMaxBlock + kThreads - 1) / kThreads;  // outputs per thread (max)
   double acc[kPer];
 #pragma unroll
@@ -271,7 +275,18 @@ __global__ __launch_bounds__(kThreads) void k_lob_cgemm(LobParams p, int64_t ld,
       const int rr = t / kCgK, kk = t % kCgK;
       s_a[rr][kk] = A[(r0 + rr) * ld + k0 + kk];
     }
-    for (int t = threadIdx.x; t < kCgK * m; t += kThreads) s_r[t / m][t % m] = R[(k0 + t / m) * m + t % m];
+    for (int t = threadIdx.x; t < kCgK * m; t += kThreads) {
+      const double* src = R + (k0 + t / m) * m + t % m;
+      double r = 0.0;
+      for (int q = 0; q < p.agg_parts; q += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = src[min(q + u, p.agg_parts - 1) * ld * m];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) r += q + u < p.agg_parts ? x[u] : 0.0;
+      }
+      s_r[t / m][t % m] = r;
+    }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
@@ -1418,12 +1433,12 @@ struct LobWork {
   double* C;
   double* Z;
   double* Gp;  // [nvar][2][2m][2m] Gram blocks of the next X and P (upper triangles)
-  double* rc;  // two-level: [nvar][ld][m] restricted residuals and coarse solutions
+  double* rc;  // two-level: [nvar][agg_parts][ld][m] restricted residuals and [nvar][ld][m] coarse solutions
   double* zc;
   int64_t bytes;
 };
 
-LobParams make_params(const fe_bsr* K, const fe_lobpcg_opts* o) {
+LobParams make_params(const fe_bsr* K, const fe_lobpcg_opts* o, int64_t n_agg = 0) {
   LobParams p{};
   p.nb = K->n_brows;
   p.n = K->n_brows * K->dof;
@@ -1443,6 +1458,15 @@ LobParams make_params(const fe_bsr* K, const fe_lobpcg_opts* o) {
   chunks = std::max<int64_t>(8, std::min<int64_t>(chunks, ceil_div(p.n, 64)));
   p.nchunk_g = (int)std::max<int64_t>(1, chunks);
   p.nchunk_r = (int)std::max<int64_t>(1, std::min<int64_t>(256, ceil_div(p.nb, 64)));
+  // Two-level: a residual chunk is a run of aggregates, or one of up to 16 equal parts of one where there are
+  // fewer aggregates than chunks: 20^3 cubes with 8 aggregates, 12 columns, 4 variants took 182 us with a
+  // workgroup per aggregate (78 with 1,024 threads in it) and take 28 in parts, and k_lob_cgemm, which adds
+  // the parts up, 20 us instead of 16.  Not a matter of n_variants: a variant's sums are the same in every call.
+  p.agg_parts = 1;
+  if (n_agg > 0) {
+    p.agg_parts = (int)std::max<int64_t>(1, std::min<int64_t>(16, p.nchunk_r / n_agg));
+    p.nchunk_r = (int)std::min<int64_t>(p.nchunk_r, n_agg) * p.agg_parts;
+  }
   return p;
 }
 
@@ -1465,7 +1489,7 @@ LobWork layout_lob(char* base, const LobParams& p, int64_t ld = 0) {
   w.Z = (double*)take(nv * NS * NS * (int64_t)sizeof(double));
   w.Gp = (double*)take(nv * 2 * 4 * (int64_t)p.m * p.m * (int64_t)sizeof(double));
   if (ld > 0) {
-    w.rc = (double*)take(nv * ld * p.m * (int64_t)sizeof(double));
+    w.rc = (double*)take(nv * p.agg_parts * ld * p.m * (int64_t)sizeof(double));
     w.zc = (double*)take(nv * ld * p.m * (int64_t)sizeof(double));
   }
   w.bytes = off;
@@ -1510,12 +1534,11 @@ void launch_lob_coarse(hipStream_t st, const LobParams& p, const LobCoarse& cc, 
 template <int D, int LAYOUT>
 int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
                const uint8_t* fixed, double* X, double* lam, double* res, int32_t* iters,
-               int32_t* vstatus, const LobWork& w, LobParams p, const fe_lobpcg_opts* o,
+               int32_t* vstatus, const LobWork& w, const LobParams& p, const fe_lobpcg_opts* o,
                fe_lobpcg_stats* stats, const LobCoarse& cc) {
   hipStream_t st = h->stream;
   const int nv = p.nvar;
-  if (cc.C) p.nchunk_r = (int)std::min<int64_t>(p.nchunk_r, cc.C->n_agg);  // no chunk without an aggregate
-  if (cc.C) FE_CHECK_HIP(hipMemsetAsync(w.rc, 0, (size_t)nv * cc.ld * p.m * sizeof(double), st));
+  if (cc.C) FE_CHECK_HIP(hipMemsetAsync(w.rc, 0, (size_t)nv * p.agg_parts * cc.ld * p.m * sizeof(double), st));
   const dim3 gvar((unsigned)ceil_div(nv, 64));
   hipLaunchKernelGGL(k_lob_init, gvar, dim3(64), 0, st, p, w.st);
   FE_CHECK_LAUNCH();
@@ -1586,12 +1609,8 @@ int run_lobpcg(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* T,
       }
       constexpr int NC = D == 3 ? 6 : D == 2 ? 3 : 1;
       if (cc.C) {
-        // an aggregate is one workgroup's: 1,024 threads where they all find a node of an average one (20^3
-        // cubes, 4 variants, 12 columns: 182 us with 256 threads, 78 with 1,024)
-        auto resid = p.nb / cc.C->n_agg >= 1024 / p.m ? k_lob_resid_agg<D, NC, 1024> : k_lob_resid_agg<D, NC, kThreads>;
-        const int nt = p.nb / cc.C->n_agg >= 1024 / p.m ? 1024 : kThreads;
-        hipLaunchKernelGGL(resid, gres, dim3(nt), 0, st, p, *cc.C, cc.ld, T, o->t_stride, fixed, w.st, w.blk,
-                           w.rpart, w.rc);
+        hipLaunchKernelGGL((k_lob_resid_agg<D, NC>), gres, dim3(kThreads), 0, st, p, *cc.C, cc.ld, T,
+                           o->t_stride, fixed, w.st, w.blk, w.rpart, w.rc);
         launch_lob_coarse<D, NC>(st, p, cc, w);
       } else {
         hipLaunchKernelGGL((k_lob_resid<D>), gres, dim3(kThreads), 0, st, p, T, o->t_stride, fixed,
@@ -1660,7 +1679,7 @@ int lobpcg_common(fe_handle* h, const fe_bsr* K, const fe_bsr* M, const double* 
   FE_REQUIRE(o->k_stride >= 0 && o->m_stride >= 0 && o->t_stride >= 0, "%s: strides must be non-negative",
              who);
   *stats = fe_lobpcg_stats{};
-  const LobParams p = make_params(K, o);
+  const LobParams p = make_params(K, o, cc.C ? cc.C->n_agg : 0);
   const LobWork w = layout_lob((char*)work, p, cc.ld);
   FE_REQUIRE(work_bytes >= w.bytes, "%s: workspace too small (%lld < %lld)", who, (long long)work_bytes,
              (long long)w.bytes);
@@ -1707,7 +1726,7 @@ extern "C" int fe_lobpcg_coarse_workspace(fe_handle* h, const fe_bsr* K, const f
   rc = check_lob_coarse(K, C, "fe_lobpcg_coarse_workspace");
   if (rc) return rc;
   FE_REQUIRE(bytes, "fe_lobpcg_coarse_workspace: null argument");
-  *bytes = layout_lob(nullptr, make_params(K, o), fe_coarse_ld(C->n_agg * C->nc)).bytes;
+  *bytes = layout_lob(nullptr, make_params(K, o, C->n_agg), fe_coarse_ld(C->n_agg * C->nc)).bytes;
   return FE_OK;
 }
 

@@ -79,35 +79,35 @@ class Context:
             t = t.to(dtype)
         return t.to(self.torch_device)
 
-    #: arrays up to this size share one copy to the device: a copy costs the host about 17 us whatever its
-    #: size, and collecting 64 KiB about 5
-    PACK_BYTES = 64 * 1024
-
-    def tensors(self, *arrays):
-        """``tensor`` of each array (None stays None), the small ones in one copy."""
-        arrays = [None if a is None else np.ascontiguousarray(a) for a in arrays]
-        small = [k for k, a in enumerate(arrays) if a is not None and 0 < a.nbytes <= self.PACK_BYTES]
-        out = [None if a is None or k in small else self.tensor(a) for k, a in enumerate(arrays)]
-        ends = np.cumsum([-(-arrays[k].nbytes // 512) * 512 for k in small])  # aligned as allocations are
-        if small:
-            host = np.empty(int(ends[-1]), dtype=np.uint8)
-            views = []
-            for k, end in zip(small, ends):
-                a = arrays[k]
-                off = int(end) - (-(-a.nbytes // 512) * 512)
-                host[off:off + a.nbytes] = a.reshape(-1).view(np.uint8)
-                views.append((k, off, a))
-            dev = self.tensor(host)
-            for k, off, a in views:
-                dtype = torch.as_tensor(a).dtype
-                out[k] = dev[off:off + a.nbytes].view(dtype).reshape(a.shape)
-        return out
-
     def empty(self, n, dtype=torch.float64):
         return torch.empty(int(n), dtype=dtype, device=self.torch_device)
 
     def zeros(self, n, dtype=torch.float64):
         return torch.zeros(int(n), dtype=dtype, device=self.torch_device)
+
+
+#: arrays up to this size share one copy to the device: a copy costs the host about 17 us whatever its
+#: size, and collecting 64 KiB about 5
+PACK_BYTES = 64 * 1024
+
+
+def upload(ctx, *arrays):
+    """``ctx.tensor`` of each array (None stays None), the small ones in one copy."""
+    arrays = [None if a is None else np.ascontiguousarray(a) for a in arrays]
+    limit = PACK_BYTES if isinstance(ctx, Context) else 0  # (a stand-in's tensor() takes arrays as they are)
+    small = [k for k, a in enumerate(arrays) if a is not None and 0 < a.nbytes <= limit]
+    out = [None if a is None or k in small else ctx.tensor(a) for k, a in enumerate(arrays)]
+    if small:
+        sizes = [-(-arrays[k].nbytes // 512) * 512 for k in small]  # aligned as allocations are
+        starts = np.cumsum([0] + sizes)
+        host = np.empty(int(starts[-1]), dtype=np.uint8)
+        for k, off in zip(small, starts):
+            host[off:off + arrays[k].nbytes] = arrays[k].reshape(-1).view(np.uint8)
+        dev = ctx.tensor(host)
+        for k, off in zip(small, starts):
+            a = arrays[k]
+            out[k] = dev[int(off):int(off) + a.nbytes].view(torch.as_tensor(a).dtype).reshape(a.shape)
+    return out
 
 
 # ------------------------------------------------------------------------------------------------
@@ -230,8 +230,8 @@ class DeviceMesh:
             mats = mat('E'), mat('nu'), None
         else:
             mats = mat('mu'), None, None
-        (self.x, self.y, self.z, self.conn, self.mat0, self.mat1, self.mat2, self.rho) = ctx.tensors(
-            coords[:, 0], coords[:, 1], coords[:, 2] if coords.shape[1] > 2 else None, conn.T, *mats, mat('rho'))
+        (self.x, self.y, self.z, self.conn, self.mat0, self.mat1, self.mat2, self.rho) = upload(
+            ctx, coords[:, 0], coords[:, 1], coords[:, 2] if coords.shape[1] > 2 else None, conn.T, *mats, mat('rho'))
 
     def struct(self) -> _hip.FeMesh:
         return _hip.FeMesh(self.kind_id, self.plane_mode, self.n_elem, self.n_nodes, _vp(self.x),
@@ -270,8 +270,8 @@ class DeviceGraph:
         bdiag = np.full(max(self.n_nodes, 1), -1, dtype=np.int32)
         q = np.nonzero(pat.bcol == rows)[0]
         bdiag[rows[q]] = q
-        (self.bptr, self.bcol, self.inc_ptr, self.inc, self.bseg_ptr, self.bseg, self.bdiag) = ctx.tensors(
-            pat.bptr, pat.bcol, pat.inc_ptr, pat.inc, pat.bseg_ptr, pat.bseg.view(np.int16), bdiag)
+        (self.bptr, self.bcol, self.inc_ptr, self.inc, self.bseg_ptr, self.bseg, self.bdiag) = upload(
+            ctx, pat.bptr, pat.bcol, pat.inc_ptr, pat.inc, pat.bseg_ptr, pat.bseg.view(np.int16), bdiag)
         self._conn = None
         self.set_schedule(pat.blk, pat.max_inc)
         self._padded = None
@@ -354,8 +354,8 @@ class DeviceGraph:
             hdr[:, 4], hdr[:, 5] = p.inc_ptr[n0], p.inc_ptr[n1] - p.inc_ptr[n0]
             hdr[:, 6], hdr[:, 7] = B0, B1 - B0
             hdr[:, 8], hdr[:, 9] = p.bseg_ptr[B0], p.bseg_ptr[B1] - p.bseg_ptr[B0]
-        self.blk, self.welem_ptr, self.welem, self.inc_sa, self.wg_hdr = self.ctx.tensors(
-            blk, wptr, welem if welem.size else np.zeros(1, np.int32),
+        self.blk, self.welem_ptr, self.welem, self.inc_sa, self.wg_hdr = upload(
+            self.ctx, blk, wptr, welem if welem.size else np.zeros(1, np.int32),
             (inc_sa if inc_sa.size else np.zeros(1, np.uint16)).view(np.int16),
             hdr.reshape(-1) if hdr.size else np.zeros(12, np.int32))
         self._hdr_host = hdr
@@ -451,7 +451,7 @@ class PaddedGraph:
             pptr, bcol, src = pad_pattern(optr, ocol, a)
             src[src >= 0] = osrc[src[src >= 0]]
         self.nnzb = int(pptr[-1])
-        self.bptr, self.bcol, self.src_block = self.ctx.tensors(pptr, bcol, src)
+        self.bptr, self.bcol, self.src_block = upload(self.ctx, pptr, bcol, src)
 
 
 def ordered_graph(graph, order: np.ndarray) -> PaddedGraph:
@@ -660,8 +660,8 @@ class DeviceCoarse:
         if cs.agg_seg is not None:
             seg = cs.agg_seg, cs.seg_of_agg if cs.seg_of_agg.size else np.zeros(1, np.int32), cs.blk_ofs
         (self.node_agg, self.agg_ptr, self.agg_nodes, self.pair_ptr, self.pair_ij, self.pair_q, self.pair_row,
-         self.P, self.xhat, self.fixed_bits, self.T, self.agg_seg, self.seg_of_agg, self.blk_ofs) = ctx.tensors(
-            cs.node_agg, cs.agg_ptr, cs.agg_nodes, cs.pair_ptr, cs.pair_ij, cs.pair_q, cs.pair_row,
+         self.P, self.xhat, self.fixed_bits, self.T, self.agg_seg, self.seg_of_agg, self.blk_ofs) = upload(
+            ctx, cs.node_agg, cs.agg_ptr, cs.agg_nodes, cs.pair_ptr, cs.pair_ij, cs.pair_q, cs.pair_row,
             cs.P.reshape(-1), xh.reshape(-1), cs.fixed_bits, cs.T.reshape(-1), *seg)
         self.P32 = _to_f32(ctx, self.P)
         self.xhat32 = _to_f32(ctx, self.xhat)

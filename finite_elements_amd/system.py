@@ -137,7 +137,7 @@ class FESystem:
         mask[fixed_dofs] = 1
         if values is not None:
             g[fixed_dofs] = np.asarray(values, dtype=np.float64)
-        return tuple(self.ctx.tensors(mask, g))
+        return tuple(device.upload(self.ctx, mask, g))
 
     def prepare(self, K: BsrMatrix, fixed: torch.Tensor, g: torch.Tensor, f: torch.Tensor,
                 coarse=None):

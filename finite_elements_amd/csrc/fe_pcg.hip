@@ -22,6 +22,9 @@
 // segment restarts from the true residual; ten updates without progress stop it as not converged.
 // Every reduction is a fixed-order sum (run-to-run bitwise reproducible).  The host polls a status
 // word one chunk behind; a chunk can be replayed from a captured HIP graph.
+//
+// One system small enough for the chip is solved in one launch instead (fe_pcg_team.h, with the same
+// arithmetic); the kernels here take larger systems, batches and profiled runs.
 #include <algorithm>
 #include <vector>
 

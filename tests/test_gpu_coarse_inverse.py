@@ -1,11 +1,13 @@
 """The inverse of the coarse operator at the edges of its blocking: orders below, at and above a block of 16 or
-64, one panel and several (an odd and an even number of them), dense and block-diagonal."""
+64, one panel and several (an odd and an even number of them), dense and block-diagonal, and the block-diagonal
+correction with it."""
 
 import numpy as np
 import pytest
 
 from finite_elements_amd import meshgen
-from tests.test_gpu_coarse import _setup
+from oracle import coarse as oc
+from tests.test_gpu_coarse import _host_matrix, _setup
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +39,9 @@ def test_inverse_orders(ctx, n, target, order):
         A = seg.operator(KD, invert=False)[0].cpu().numpy()[:k * k].reshape(k, k)
         inv, inv32 = seg.operator(KD, invert=True)
         _check(inv.cpu().numpy()[:k * k].reshape(k, k), inv32.cpu().numpy()[:k * k].reshape(k, k), A)
+        ref, P = oc.coarse_operator(seg.host, _host_matrix(KD))
+        r = np.random.default_rng(order).standard_normal(P.shape[0])
+        want = P @ np.linalg.solve(ref, P.T @ r)
+        u = s.ctx.tensor(np.zeros(P.shape[0]))
+        seg.apply(inv, s.ctx.tensor(r), u)
+        assert np.abs(u.cpu().numpy() - want).max() <= 1e-10 * np.abs(want).max()

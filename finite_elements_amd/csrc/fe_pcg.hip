@@ -718,8 +718,8 @@ struct Work {
   uint64_t* flags;  // the team's arrival flags, then its abort word
   uint64_t* ut;     // its messages: u, and the partial dots
   uint64_t* pt;
-  char* ring;       // its moments, and B = T A_c^-1 T^T (two-level)
-  void* binv;
+  char* ring;       // its shares of P^T w, and A_c^-1 in FP32 (two-level)
+  float* ainv32;
   fe_pcg_seg_stats* seg_stats;
   void* r;
   void* u;
@@ -765,7 +765,7 @@ Work layout_work(char* base, int64_t nb, int dof, int elem, int nseg, int64_t nt
   w.pt = (uint64_t*)take(team ? 12 * kTeamCopies * std::max<int64_t>(1, ntiles) * (int64_t)sizeof(uint64_t) : 0);
   const bool team_co = team && n_coarse > 0 && n_coarse <= kTeamMaxCoarse;
   w.ring = (char*)take(team_co ? kTeamRing * team_region(std::min<int64_t>(ntiles, 256), ntiles, n_coarse, 6, 8) : 0);
-  w.binv = take(team_co ? n_coarse * fe_coarse_ld(n_coarse) * (int64_t)sizeof(double) : 0);
+  w.ainv32 = (float*)take(team_co ? n_coarse * fe_coarse_ld(n_coarse) * (int64_t)sizeof(float) : 0);
   w.seg_stats = (fe_pcg_seg_stats*)take(nseg * (int64_t)sizeof(fe_pcg_seg_stats));
   w.r = take(n * elem);
   w.u = take(n * elem);
@@ -872,8 +872,9 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
     a.xhat = sizeof(T) == 4 ? (const void*)C->xhat32 : (const void*)C->xhat;
     a.fixed_bits = C->fixed_bits;
     a.n_agg = (int32_t)C->n_agg;
-    a.ldb = fe_coarse_ld(C->n_agg * NC);
-    a.B = w.binv;
+    a.Tm = C->T;
+    a.lda = fe_coarse_ld(C->n_agg * NC);
+    a.Ainv = sizeof(T) == 4 ? (const void*)w.ainv32 : pb.Ainv64;
     a.ring = w.ring;
     a.region = team_region(ceil_div(a.ntiles, S), a.ntiles, pb.C->n_agg, NC, (int)sizeof(T));
   }
@@ -886,9 +887,11 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   FE_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock * S, (size_t)lds));
   if (grid > (int64_t)per_cu * h->num_cus) return FE_OK;
   FE_CHECK_HIP(hipMemsetAsync(w.flags, 0, (kTeamMaxTiles + 1) * sizeof(uint64_t), st));
-  if constexpr (CO)
-    hipLaunchKernelGGL((k_team_binv<T, NC>), dim3((unsigned)ceil_div(pb.C->n_agg * pb.C->n_agg, 64)), dim3(64), 0, st,
-                       (int32_t)pb.C->n_agg, (const double*)pb.Ainv64, a.ldb, pb.C->T, (T*)w.binv);
+  if constexpr (CO && sizeof(T) == 4) {
+    const int64_t n = pb.C->n_agg * NC * a.lda;
+    hipLaunchKernelGGL(k_team_cast, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, n, (const double*)pb.Ainv64,
+                       w.ainv32);
+  }
   void* args[] = {&a};
   hipError_t e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)grid), dim3(kBlock * S), args, (unsigned)lds, st);
   if (e != hipSuccess) {

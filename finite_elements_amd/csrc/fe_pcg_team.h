@@ -22,13 +22,17 @@
 // Two-level preconditioner (CO): the node rows are numbered aggregate by aggregate (order), so that a
 // workgroup's rows touch few aggregates.  The correction P A_c^-1 P^T r is carried by the recurrence of r:
 // with z, zeta and y the corrections of r, s and w, s = w + beta s gives zeta = y + beta zeta and
-// r -= alpha s gives z -= alpha zeta, so an iteration needs P^T w only.  Every tile sums the rigid-body
-// moments of its rows of w by aggregate and hands them over with its partial dots; every workgroup adds
-// all of them up and applies the rows of B = T A_c^-1 T^T that its own aggregates need.  The correction costs no
-// further meeting (launched: three kernels per iteration).  The reliable updates form z, zeta and y anew.
-// All workgroups read all moments, a few KB that message words and agent-scope loads would fetch from
+// r -= alpha s gives z -= alpha zeta, so an iteration needs P^T w only.  Every tile sums its rows' share of
+// P^T w by aggregate and hands it over with its partial dots; every workgroup adds all of them up and applies
+// the rows of A_c^-1 that its own aggregates need.  The correction costs no further meeting (launched:
+// three kernels per iteration).  The reliable updates form z, zeta and y anew.
+// Shares, z, zeta and y are in the coarse space's orthonormal basis (P = Z T): the rigid-body moments and
+// motions on the other side of T stay in FP64 inside a tile or an aggregate.  An aggregate of two nodes, or of
+// nodes on a line, has T entries of 1e8, and a product such as T A_c^-1 T^T, a moment rounded to FP32 or a
+// recurrence in the motions would lose the correction in them.
+// All workgroups read all shares, a few KB that message words and agent-scope loads would fetch from
 // memory once per workgroup (450^2 magnetostatics, 199 workgroups: 16 us per iteration).  So here the
-// moments and dots are stored first, by agent-scope stores, then a flag, and read by plain loads, which
+// shares and dots are stored first, by agent-scope stores, then a flag, and read by plain loads, which
 // the workgroups of an XCD share through its L2.  That is sound because a meeting's region of memory has not
 // been read since the last invalidation: the regions are a ring of kTeamRing, and every wavefront
 // invalidates (agent-scope acquire fence) before it reads the ring's first region; a workgroup's part of a
@@ -50,8 +54,8 @@ namespace {
 constexpr int kTeamMaxTiles = 1024;
 constexpr int kTeamSpins = 1 << 21;  // polls of about a microsecond
 constexpr int kTeamCopies = 8;  // of the partial dots: a workgroup reads copy blockIdx.x % 8
-constexpr int kTeamMaxCoarse = 1536;  // coarse DOF: every workgroup holds all their moments in LDS
-constexpr int kTeamRing = 64;   // regions of the moments' ring
+constexpr int kTeamMaxCoarse = 1536;  // coarse DOF: every workgroup holds all of P^T w in LDS
+constexpr int kTeamRing = 64;   // regions of the shares' ring
 constexpr int kTeamLds = 144 * 1024;  // dynamic LDS of a workgroup, of the CU's 160 KB
 
 struct TeamArgs {
@@ -75,56 +79,31 @@ struct TeamArgs {
   int32_t chunk;
   int64_t max_chunks;
   // two-level: node rows by aggregate (row i of the iteration matrix is node order[i]), the aggregates'
-  // row ranges, their nodes' x^ and constraint bits, B (iteration precision, leading dimension ldb) and
-  // the ring of kTeamRing regions of region bytes
+  // row ranges, their nodes' x^ and constraint bits, their T, A_c^-1 (iteration precision, leading
+  // dimension lda) and the ring of kTeamRing regions of region bytes
   const int32_t *order, *agg_ptr, *node_agg;
   const void* xhat;
   const uint8_t* fixed_bits;
-  const void* B;
-  int64_t ldb;
+  const double* Tm;
+  const void* Ainv;
+  int64_t lda;
   int32_t n_agg;
   char* ring;
   int64_t region;
 };
 
-// B = T A_c^-1 T^T by blocks (I, J) of coarse DOF: the correction in rigid-body moments and motions.
-template <typename T, int NC>
-__global__ __launch_bounds__(64) void k_team_binv(int32_t n_agg, const double* __restrict__ Ainv, int64_t ld,
-                                                  const double* __restrict__ Tm, T* __restrict__ B) {
-  const int64_t t = blockIdx.x * (int64_t)64 + threadIdx.x;
-  if (t >= (int64_t)n_agg * n_agg) return;
-  const int64_t I = t / n_agg, J = t % n_agg;
-  double a[NC][NC], q[NC][NC];
-#pragma unroll
-  for (int x = 0; x < NC; ++x)
-#pragma unroll
-    for (int y = 0; y < NC; ++y) a[x][y] = Ainv[(I * NC + x) * ld + J * NC + y];
-#pragma unroll
-  for (int x = 0; x < NC; ++x)
-#pragma unroll
-    for (int y = 0; y < NC; ++y) {
-      double v = 0.0;
-#pragma unroll
-      for (int k = 0; k < NC; ++k) v += a[x][k] * Tm[(J * NC + y) * NC + k];
-      q[x][y] = v;
-    }
-#pragma unroll
-  for (int x = 0; x < NC; ++x)
-#pragma unroll
-    for (int y = 0; y < NC; ++y) {
-      double v = 0.0;
-#pragma unroll
-      for (int k = 0; k < NC; ++k) v += Tm[(I * NC + x) * NC + k] * q[k][y];
-      B[(I * NC + x) * ld + J * NC + y] = (T)v;
-    }
+// A_c^-1 in FP32.
+__global__ __launch_bounds__(256) void k_team_cast(int64_t n, const double* __restrict__ in, float* __restrict__ out) {
+  const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (t < n) out[t] = (float)in[t];
 }
 
-// A region of the ring: workgroup b's three partial dots, then the moments of its parts, the first of them
+// A region of the ring: workgroup b's three partial dots, then its parts, the first of them
 // part q0; its place leaves whole cache lines to the workgroups before it.
 inline __host__ __device__ int64_t team_part(int64_t b, int64_t q0, int NC, int elem) {
   return 128 * (2 * b + q0 * NC * elem / 128);
 }
-constexpr int kTeamDots = 32;  // bytes of the dots ahead of the moments
+constexpr int kTeamDots = 32;  // bytes of the dots ahead of the parts
 
 // Dynamic LDS of a workgroup: the parts beside u's, which take the rest.
 struct TeamLds {
@@ -315,13 +294,13 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     __syncthreads();
   }
   const int nr = s_scan[NT - 1];  // remote rows
-  // two-level: behind the remote rows' u, the coarse vectors of the workgroup's aggregates
+  // two-level: behind the remote rows' u, the coarse vectors and T of the workgroup's aggregates
   int g0 = 0, ng = 0;
   if constexpr (CO) {
     g0 = a.node_agg[a.order[wr0]];
     ng = (wr1 > wr0 ? a.node_agg[a.order[wr1 - 1]] : g0) - g0 + 1;
   }
-  const int co_rows = (3 * ng * NC * 8 + 16 + D * (int)sizeof(T) - 1) / (D * (int)sizeof(T));  // in rows of u
+  const int co_rows = ((4 + NC) * ng * NC * 8 + 16 + D * (int)sizeof(T) - 1) / (D * (int)sizeof(T));  // in rows of u
   const bool fits = nr + (CO ? co_rows : 0) <= a.lds_remote;
   int at = s_scan[threadIdx.x] - count;
   for (int k = w0; k < w1; ++k) {
@@ -579,7 +558,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   // ---- coarse correction (CO) -----------------------------------------------------------------------
   const int n_c = CO ? a.n_agg * NC : 0;
   double* zc = (double*)(s_dyn + (((size_t)(S * R + nr) * D * sizeof(T) + 15) & ~(size_t)15));
-  double *ze = zc + ng * NC, *yc = ze + ng * NC;
+  double *ze = zc + ng * NC, *yc = ze + ng * NC, *ym = yc + ng * NC, *tl = ym + ng * NC;
   int tg0 = 0, tg1 = -1;
   if constexpr (CO) {
     // the tile's parts: its aggregates, from that of the row before it (an empty part where the tile starts
@@ -595,8 +574,10 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) xl[(i - wr0) * 3 + c] = ((const T*)a.xhat)[node * 3 + c];
     }
+    if (fits)
+      for (int e = threadIdx.x; e < ng * NC * NC; e += NT) tl[e] = a.Tm[(int64_t)g0 * NC * NC + e];
   }
-  int32_t la[kPasses];  // first of the node's aggregate's entries in zc, or -1 where the DOF is constrained
+  int32_t la[kPasses];  // first of the node's aggregate's entries in ym, or -1 where the DOF is constrained
 #pragma unroll
   for (int ps = 0; ps < kPasses; ++ps) {
     la[ps] = -1;
@@ -618,16 +599,16 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     for (int g = threadIdx.x; g <= a.n_agg; g += NT) aggp[g] = a.agg_ptr[g];
   constexpr int kParts = 2;
   int turn = 0;  // region of the ring
-  // the rows of B that this workgroup applies, in LDS behind the remote rows where they fit
-  const T* Brows = (const T*)a.B + (int64_t)g0 * NC * a.ldb;
-  int64_t ldb = a.ldb;
+  // the rows of A_c^-1 that this workgroup applies, in LDS behind the remote rows where they fit
+  const T* Arows = (const T*)a.Ainv + (int64_t)g0 * NC * a.lda;
+  int64_t lda = a.lda;
   if constexpr (CO) {
     if (fits && (int64_t)ng * NC * n_c <= (int64_t)(a.lds_remote - nr - co_rows) * D) {
-      T* Bl = (T*)(yc + ng * NC);
+      T* Al = (T*)(tl + ng * NC * NC);
       for (int q = (int)threadIdx.x / 64; q < ng * NC; q += NT / 64)
-        for (int c = wl; c < n_c; c += 64) Bl[q * n_c + c] = Brows[q * ldb + c];
-      Brows = Bl;
-      ldb = n_c;
+        for (int c = wl; c < n_c; c += 64) Al[q * n_c + c] = Arows[q * lda + c];
+      Arows = Al;
+      lda = n_c;
     }
   }
   auto coarse_rows = [&](const T* v) {
@@ -637,8 +618,8 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       if (lane < D && i < row1) wl_[(i - wr0) * D + lane] = v[ps];
     }
   };
-  // A meeting of all for the moments of the rows in wl_ and, if v3, the dots' wavefront sums in s_red (both
-  // behind a barrier): c in cm, the dots' sums over the workgroups' wavefronts in s_sum.
+  // A meeting of all for P^T of the rows in wl_ and, if v3, the dots' wavefront sums in s_red (both
+  // behind a barrier): P^T w in cm, the dots' sums over the workgroups' wavefronts in s_sum.
   auto coarse_meet = [&](bool dots) {
     char* region = a.ring + turn * a.region;
     if (++turn == kTeamRing) turn = 0;
@@ -676,12 +657,11 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
           m[0] += rv[0];
         }
       }
+      // T^T of the moments (an empty part may be of the aggregate before the workgroup's first)
       double mine_c = 0.0;
+      const double* tg = tl + (max(g, g0) - g0) * NC * NC + min(wl, NC - 1);
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const double t = wave_sum(m[c]);
-        mine_c = wl == c ? t : mine_c;
-      }
+      for (int c = 0; c < NC; ++c) mine_c += tg[c * NC] * wave_sum(m[c]);
       if (wl < NC) put((T*)(mine + kTeamDots) + (tile + g - q0) * NC + wl, (T)mine_c);
     }
     if (dots && threadIdx.x < 3) {
@@ -732,10 +712,10 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     __syncthreads();
     return s_fail == 0;
   };
-  // (behind a barrier) out = B c for the workgroup's aggregates, one wavefront per row
+  // (behind a barrier) out = A_c^-1 cm for the workgroup's aggregates, one wavefront per row
   auto coarse_apply_rows = [&](double* out) {
     for (int q = (int)threadIdx.x / 64; q < ng * NC; q += NT / 64) {
-      const T* row = Brows + q * ldb;
+      const T* row = Arows + q * lda;
       double v = 0.0;
 #pragma unroll 8
       for (int c = wl; c < n_c; c += 64) v += (double)row[c] * cm[c];
@@ -743,7 +723,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       if (wl == 0) out[q] = v;
     }
   };
-  // out = B P^T v, a meeting of its own (reliable updates)
+  // out = A_c^-1 P^T v, a meeting of its own (reliable updates)
   auto coarse_round = [&](const T* v, double* out) {
     coarse_rows(v);
     __syncthreads();
@@ -752,13 +732,29 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     __syncthreads();
     return s_fail == 0;
   };
-  // u += the rigid-body motion z of the node's aggregate, on free DOFs
+  // The rigid-body motions ym = T z of the workgroup's aggregates, z = zc after step(entry) has brought it up to
+  // date; an aggregate's entries are neighbouring lanes'.
+  auto coarse_motions = [&](auto step) {
+    constexpr int L = NC == 6 ? 8 : NC == 3 ? 4 : 1;
+    for (int e = threadIdx.x; e < ng * L; e += NT) {
+      const int q = e / L * NC + min(e % L, NC - 1);
+      const bool on = e % L < NC;
+      const double z = on ? step(q) : 0.0;
+      const double* t = tl + q * NC;
+      double y = 0.0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) y += t[k] * (L == 1 ? z : __shfl(z, k, L));
+      if (on) ym[q] = y;
+    }
+    __syncthreads();
+  };
+  // u += the rigid-body motion of the node's aggregate, on free DOFs
   auto coarse_add = [&]() {
 #pragma unroll
     for (int ps = 0; ps < kPasses; ++ps) {
       if (la[ps] < 0) continue;
       const int l = team_here(my_row) + ps * kRows - wr0;
-      const double* y = zc + la[ps];
+      const double* y = ym + la[ps];
       double du = y[lane];
       if constexpr (D == 3) {
         // lane 0: z w_y - y w_z, lane 1: x w_z - z w_x, lane 2: y w_x - x w_y
@@ -824,6 +820,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       }
       if constexpr (CO) {
         if (!coarse_round(rk, zc)) { alive = false; break; }
+        coarse_motions([&](int q) { return zc[q]; });
       }
       precond();
       if constexpr (CO) coarse_add();
@@ -900,11 +897,10 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       const double alpha = st.alpha;
       const T alpha_t = (T)alpha, beta = (T)st.beta;
       if constexpr (CO) {
-        for (int q = threadIdx.x; q < ng * NC; q += NT) {
+        coarse_motions([&](int q) {
           ze[q] = yc[q] + st.beta * ze[q];
-          zc[q] -= alpha * ze[q];
-        }
-        __syncthreads();
+          return zc[q] -= alpha * ze[q];
+        });
       }
 #pragma unroll
       for (int ps = 0; ps < kPasses; ++ps) {

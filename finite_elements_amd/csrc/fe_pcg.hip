@@ -38,7 +38,8 @@ struct PcgState {
   double alpha, beta, gamma, gamma_prev;
   double rr, rr_ref, rr_true, bb;
   double tol2bb, ru_delta2, rr_best;
-  double rgamma, ralpha;  // reciprocals of gamma and alpha, formed off the next sums' critical path
+  // reciprocals of gamma (times the power of two up) and alpha, formed off the next sums' critical path
+  double rgamma, ralpha, up;
   int32_t iter, max_iter;
   int32_t done;     // 0 running, 1 converged, 2 iteration limit / stagnation, 3 breakdown
   int32_t need_ru;  // 1: reliable update / true-residual check requested
@@ -315,12 +316,21 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(const Tile* __restrict__ til
 
 // What the scalars of the next iteration are formed from, beside the sums (read ahead of them).
 struct CgIn {
-  double gamma, rgamma, ralpha, tol2bb, ru_delta2, rr_ref;
+  double gamma, rgamma, ralpha, up, tol2bb, ru_delta2, rr_ref;
   int32_t iter, max_iter, mixed, ru_pending;
 };
 __device__ inline CgIn cg_in(const PcgState* s) {
-  return CgIn{s->gamma, s->rgamma, s->ralpha, s->tol2bb, s->ru_delta2, s->rr_ref,
+  return CgIn{s->gamma, s->rgamma, s->ralpha, s->up, s->tol2bb, s->ru_delta2, s->rr_ref,
               s->iter + 1, s->max_iter, s->mixed, s->ru_pending};
+}
+
+// rgamma and ralpha for alpha = gamma / den.  A subnormal gamma (right-hand sides near 1e-150) has no
+// reciprocal of its own, so a small one is scaled first.
+__device__ inline void set_recips(PcgState* s, double gamma, double den) {
+  const double up = gamma < 0x1p-960 ? 0x1p600 : 1.0;
+  s->up = up;
+  s->rgamma = 1.0 / (gamma * up);
+  s->ralpha = den / gamma;
 }
 
 // The Chronopoulos-Gear scalars for the next iteration from the sums v = (r.u, w.u, r.r), by one thread.
@@ -343,7 +353,7 @@ __device__ inline void cg_scalars(PcgState* s, const CgIn& c, const double (&v)[
   }
   const bool pending = c.ru_pending || (c.mixed && v[2] < c.ru_delta2 * c.rr_ref);
   if (pending) s->ru_pending = 1;
-  const double beta = g * c.rgamma;
+  const double beta = g * c.up * c.rgamma;
   const double den = dl - beta * g * c.ralpha;
   if (!(den > 0.0)) {
     // the recurrences lost positivity (rounding, most often in FP32): restart from the true
@@ -355,8 +365,7 @@ __device__ inline void cg_scalars(PcgState* s, const CgIn& c, const double (&v)[
   }
   s->beta = beta;
   s->alpha = g / den;
-  s->rgamma = 1.0 / g;
-  s->ralpha = den / g;
+  set_recips(s, g, den);
   // the update replaces r, u, w, s and recomputes beta and alpha from gamma_prev, as at a hand-over
   if (last && pending) s->need_ru = 1;
 }
@@ -373,8 +382,9 @@ __global__ __launch_bounds__(kRed) void k_cg_reduce(const int32_t* __restrict__ 
   const CgIn c = cg_in(s);
   // an empty asm that takes the values keeps their loads ahead of the exit (the compiler would
   // otherwise sink each one to its first use, a memory round trip apiece)
-  asm volatile("" ::"s"(t0), "s"(t1), "s"(c.gamma), "s"(c.rgamma), "s"(c.ralpha), "s"(c.tol2bb), "s"(c.ru_delta2),
-               "s"(c.rr_ref), "s"(c.iter), "s"(c.max_iter), "s"(c.mixed), "s"(c.ru_pending), "s"(ntiles), "s"(partials));
+  asm volatile("" ::"s"(t0), "s"(t1), "s"(c.gamma), "s"(c.rgamma), "s"(c.ralpha), "s"(c.up), "s"(c.tol2bb),
+               "s"(c.ru_delta2), "s"(c.rr_ref), "s"(c.iter), "s"(c.max_iter), "s"(c.mixed), "s"(c.ru_pending),
+               "s"(ntiles), "s"(partials));
   if (done | need_ru) return;
   double v[3];
   seg_sum<3>(partials, ntiles, t0, t1, v);
@@ -579,8 +589,7 @@ __device__ inline void ru_finish(PcgState* s, const double (&v)[5]) {
   s->beta = beta;
   s->alpha = g / pap;
   s->gamma = g;
-  s->rgamma = 1.0 / g;
-  s->ralpha = pap / g;
+  set_recips(s, g, pap);
   s->first = 0;
   s->rr = v[4];
   s->rr_ref = s->rr_true;
@@ -639,6 +648,7 @@ __global__ __launch_bounds__(kRed) void k_pcg_init(const int32_t* __restrict__ s
   s->gamma_prev = 1.0;
   s->rgamma = 1.0;
   s->ralpha = 1.0;
+  s->up = 1.0;
   s->rr_best = 1.0e308;
 }
 

@@ -959,6 +959,7 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
   hipStream_t st = h->stream;
   const T* M = (const T*)pb.M;
   const dim3 gt((unsigned)nt), gseg((unsigned)nseg);
+  h->pcg_path = FE_PCG_LAUNCHED;
   auto launch_init = [&]() -> int {
     hipLaunchKernelGGL((k_tile_norm<D>), gt, dim3(kBlock), 0, st, w.tiles, pb.b, w.partials);
     hipLaunchKernelGGL(k_pcg_init, gseg, dim3(kRed), 0, st, w.seg_tiles, nt, w.partials, w.st, o->tol,
@@ -972,9 +973,11 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
     bool ran = false, done = false;
     if (pb.ordered) {
       if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, &ran, &done);
+      h->pcg_path = done ? FE_PCG_ONE_LAUNCH : ran ? FE_PCG_LEFT : FE_PCG_LAUNCHED;
       return rc0 ? rc0 : done ? FE_OK : kErrTeamLeft;
     }
     if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, &ran, &done);
+    h->pcg_path = done ? FE_PCG_ONE_LAUNCH : ran ? FE_PCG_LEFT : FE_PCG_LAUNCHED;
     if (rc0 || done) return rc0;
     if (ran) rc0 = launch_init();  // the team gave up and left its state behind
     if (rc0) return rc0;
@@ -1246,6 +1249,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
   int rc = ntiles == 0 ? FE_OK
            : o->mixed  ? dispatch_dof<float>(h, pb, w, o, s)
                        : dispatch_dof<double>(h, pb, w, o, s);
+  const int32_t path = h->pcg_path;  // (the solves below overwrite it)
   fe_pcg_opts o_plain = *o;
   if (rc == kErrTeamLeft) {
     // the launched kernels finish an ordered solve in FP64, on A64 itself
@@ -1300,6 +1304,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
     }
     s->fallbacks = failed;
   }
+  h->pcg_path = ntiles == 0 ? FE_PCG_LAUNCHED : path;
   // aggregate: worst status, largest residuals, most iterations
   s->status = FE_OK;
   s->relres = 0.0;
@@ -1356,6 +1361,13 @@ extern "C" int fe_pcg(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const 
   if (A64->n_brows == 0) return FE_OK;
   const int32_t seg[2] = {0, (int32_t)A64->n_brows};
   return pcg_common(h, A64, A32, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr, "fe_pcg");
+}
+
+extern "C" int fe_pcg_path(fe_handle* h, int* path) {
+  FE_ENTER(h);
+  FE_REQUIRE(path, "fe_pcg_path: null argument");
+  *path = h->pcg_path;
+  return FE_OK;
 }
 
 extern "C" int fe_pcg_batched(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64,

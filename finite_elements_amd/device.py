@@ -822,10 +822,17 @@ class PcgSolver:
         return _hip.FePcgOpts(float(tol), int(max_iter), pc, int(self.mixed), int(self.check_every),
                               float(self.ru_delta), int(profile), int(self.graph))
 
+    def _path(self):
+        path = ctypes.c_int()
+        _hip.call('fe_pcg_path', self.ctx.h, ctypes.byref(path))
+        return path.value
+
     def solve(self, b: torch.Tensor, x: Optional[torch.Tensor] = None, tol: float = 1e-8,
               max_iter: Optional[int] = None, profile: bool = False):
-        """Solve from initial guess x (zeros if None); returns (x, info dict).  With segments, info
-        also holds per-segment arrays (iterations, status, relres, ...)."""
+        """Solve from initial guess x (zeros if None); returns (x, info dict).  info['path'] tells how
+        it ran: ``FE_PCG_LAUNCHED`` kernels, ``FE_PCG_ONE_LAUNCH``, or ``FE_PCG_LEFT`` when the one
+        launch gave up and launched kernels finished.  With segments, info also holds per-segment
+        arrays (iterations, status, relres, ...)."""
         ctx = self.ctx
         if max_iter is None:
             max_iter = max(2000, min(10 * self.A64.n, 50000))
@@ -890,7 +897,7 @@ class PcgSolver:
                 'restarts': stats.restarts,
                 'status': stats.status, 'relres': stats.relres, 'relres_rec': stats.relres_rec,
                 'bnorm': stats.bnorm, 'spmv_ms': stats.spmv_ms, 'spmv_samples': stats.spmv_samples,
-                'fallbacks': stats.fallbacks}
+                'fallbacks': stats.fallbacks, 'path': self._path()}
         if seg_info is not None:
             info['segments'] = seg_info
         return x, info

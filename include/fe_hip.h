@@ -343,6 +343,14 @@ int fe_pcg(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64, 
            const double* b, double* x, void* work, int64_t work_bytes, const fe_pcg_opts* opts,
            fe_pcg_stats* stats);
 
+/* How the handle's last PCG solve (of any of these entry points) ran in the precision it began in:
+   FE_PCG_LAUNCHED kernels for every step of every iteration, FE_PCG_ONE_LAUNCH all of it (a system that
+   fits on the chip), FE_PCG_LEFT begun in one launch, which gave up, and finished by launched kernels. */
+#define FE_PCG_LAUNCHED 0
+#define FE_PCG_ONE_LAUNCH 1
+#define FE_PCG_LEFT 2
+int fe_pcg_path(fe_handle* h, int* path);
+
 /* Batched PCG over independent segments of one block-diagonal system (replaces one spsolve per design
    variant, finite_elements/analysis.py:819-822): segment g owns node rows [seg_nodes[g],
    seg_nodes[g+1]) (host array, n_seg + 1 entries, 0 .. n_brows) and no block couples two segments.

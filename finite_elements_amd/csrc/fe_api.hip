@@ -38,6 +38,7 @@ extern "C" int fe_create(fe_handle** out, int device, void* stream) {
     return fe_set_error((int)e, "hipGetDeviceProperties: %s", hipGetErrorString(e));
   }
   h->num_cus = prop.multiProcessorCount;
+  h->pcg_spins = FE_PCG_SPINS;
   e = hipHostMalloc(&h->pinned, 4096, hipHostMallocDefault);
   if (e != hipSuccess) {
     delete h;

@@ -16,7 +16,8 @@ struct fe_handle {
   int num_cus;
   // Two pinned host slots for polling solver status without blocking the queue.
   void* pinned;
-  int32_t pcg_path;  // of the last PCG solve (fe_pcg_path)
+  int32_t pcg_path;   // of the last PCG solve (fe_pcg_path)
+  int32_t pcg_spins;  // fe_pcg_set_spins
 };
 
 int fe_set_error(int code, const char* fmt, ...);

@@ -865,6 +865,7 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   a.partials = w.partials;
   a.flags = w.flags;
   a.abort = (int32_t*)(w.flags + kTeamMaxTiles);
+  a.spins = h->pcg_spins;
   a.ut = w.ut;
   a.pt = w.pt;
   // LDS: u of the own rows, and of as many remote ones as fit beside the rest
@@ -1367,6 +1368,13 @@ extern "C" int fe_pcg_path(fe_handle* h, int* path) {
   FE_ENTER(h);
   FE_REQUIRE(path, "fe_pcg_path: null argument");
   *path = h->pcg_path;
+  return FE_OK;
+}
+
+extern "C" int fe_pcg_set_spins(fe_handle* h, int32_t spins) {
+  FE_ENTER(h);
+  FE_REQUIRE(spins >= 0, "fe_pcg_set_spins: negative bound");
+  h->pcg_spins = spins;
   return FE_OK;
 }
 

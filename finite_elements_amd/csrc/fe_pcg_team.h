@@ -43,8 +43,9 @@
 // coarse correction has the bits of the same system solved as a segment of a batch.
 //
 // The launch is cooperative (all workgroups resident, cooperative launches never side by side).  Every
-// wait is bounded: a workgroup that has polled kTeamSpins times raises `abort` and leaves, the others
-// follow at their own next wait, and the host finishes the solve with the launched kernels.
+// wait is bounded: a thread that has polled `spins` times raises `abort`, which ends every other wait, its own
+// next ones and the other workgroups', after 64 polls; a workgroup leaves at the end of the meeting, and the
+// host finishes the solve with the launched kernels.
 #pragma once
 
 #include "fe_sparse.h"
@@ -52,7 +53,6 @@
 namespace {
 
 constexpr int kTeamMaxTiles = 1024;
-constexpr int kTeamSpins = 1 << 21;  // polls of about a microsecond
 constexpr int kTeamCopies = 8;  // of the partial dots: a workgroup reads copy blockIdx.x % 8
 constexpr int kTeamMaxCoarse = 1536;  // coarse DOF: every workgroup holds all of P^T w in LDS
 constexpr int kTeamRing = 64;   // regions of the shares' ring
@@ -73,6 +73,7 @@ struct TeamArgs {
   double* partials;  // 2 x 5 arrays: meetings alternate between the halves
   uint64_t* flags;   // one per workgroup, zero before the launch
   int32_t* abort;    // zero before the launch
+  int32_t spins;     // bound of a wait, in polls of about a microsecond
   uint64_t* ut;      // u as messages: sizeof(T) / 4 words per DOF
   uint64_t* pt;      // partial dots as messages: 2 halves x kTeamCopies x 6 words x pstride
   int32_t lds_remote;  // remote node rows whose u fits in LDS
@@ -149,13 +150,14 @@ __device__ inline int32_t team_here(int32_t v) {
   return v;
 }
 
-// Poll until `ready()`; false when the bound is reached or another workgroup has given up.
+// Poll until `ready()`; false when another workgroup has given up or the bound is reached, which raises abort.
 template <typename F>
-__device__ inline bool team_poll(const int32_t* abort, F ready) {
-  for (int n = 0; n < kTeamSpins; ++n) {
+__device__ inline bool team_poll(int32_t* abort, int32_t spins, F ready) {
+  for (int32_t n = 0; n < spins; ++n) {
     if (ready()) return true;
     if ((n & 63) == 63 && ld_team(abort) != 0) return false;
   }
+  st_team(abort, 1);
   return false;
 }
 
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   auto meet_neighbours = [&]() {
     arrive();
     for (int g = lo + (int)threadIdx.x; g <= hi; g += NT)
-      if (!team_poll(a.abort, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
+      if (!team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
     __syncthreads();
     return s_fail == 0;
   };
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     if (sub == 0) {
       bool ok = true;
       for (int t = tid; t < a.ntiles; t += kBlock)
-        ok = ok && team_poll(a.abort, [&] { return ld_team(a.flags + t / S) >= epoch; });
+        ok = ok && team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + t / S) >= epoch; });
       if (!ok) s_fail = 1;
       // at most S kBlock tiles: one per workgroup of S subgroups, one workgroup per CU
       double e[S][NV];
@@ -436,7 +438,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
       for (int j = 0; j < B; ++j) {
         if (e0 + j * NT >= nr * D) break;
-        if (!team_got(m[j], TW, tag) && !team_poll(a.abort, [&] {
+        if (!team_got(m[j], TW, tag) && !team_poll(a.abort, a.spins, [&] {
 #pragma unroll
               for (int h = 0; h < TW; ++h) m[j][h] = ld_team(from[j] + h);
               return team_got(m[j], TW, tag);
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
       for (int j = 0; j < S; ++j) {
         if (tid + j * kBlock >= a.ntiles) break;
-        if (!got(j) && !team_poll(a.abort, [&] { load(j); return got(j); })) s_fail = 1;
+        if (!got(j) && !team_poll(a.abort, a.spins, [&] { load(j); return got(j); })) s_fail = 1;
 #pragma unroll
         for (int k = 0; k < 3; ++k) v[k] += team_value(m[j][k]);
       }
@@ -677,7 +679,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     } else {
       arrive();
       for (int g = threadIdx.x; g < nwg; g += NT)
-        if (!team_poll(a.abort, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
+        if (!team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
       __syncthreads();
       if (turn == 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the ring's first region, also the first time
     }

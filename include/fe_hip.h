@@ -350,6 +350,11 @@ int fe_pcg(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64, 
 #define FE_PCG_ONE_LAUNCH 1
 #define FE_PCG_LEFT 2
 int fe_pcg_path(fe_handle* h, int* path);
+/* Bound of a wait between the workgroups of a one-launch solve, in polls of about a microsecond
+   (FE_PCG_SPINS unless set).  A solve whose wait reaches it gives up and is finished by launched kernels;
+   with 0 that is the first wait of every solve. */
+#define FE_PCG_SPINS 2097152
+int fe_pcg_set_spins(fe_handle* h, int32_t spins);
 
 /* Batched PCG over independent segments of one block-diagonal system (replaces one spsolve per design
    variant, finite_elements/analysis.py:819-822): segment g owns node rows [seg_nodes[g],

@@ -32,6 +32,7 @@ FE_PC_JACOBI = 1
 FE_PCG_LAUNCHED = 0
 FE_PCG_ONE_LAUNCH = 1
 FE_PCG_LEFT = 2
+FE_PCG_WIDE = 3
 FE_PCG_SPINS = 2097152
 FE_PC_BLOCK_JACOBI = 2
 FE_COARSE_NOALLOC_MAX = 65536
@@ -160,6 +161,8 @@ SIGNATURES = {
     'fe_pcg_coarse_takes_ordered': (_int, [_P(FeBsr), _P(FeCoarse), _P(FePcgOpts), _P(_int)]),
     'fe_pcg_coarse_ordered': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _P(FeCoarse), _vp, _vp, _vp, _vp,
                                      _i64, _P(FePcgOpts), _P(FePcgStats)]),
+    'fe_pcg_coarse_one_launch': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _P(FeCoarse), _vp, _vp, _vp, _vp,
+                                        _i64, _P(FePcgOpts), _P(FePcgStats)]),
     'fe_pcg_batched_coarse_workspace': (_int, [_vp, _P(FeBsr), _i32, _vp, _P(FeCoarse), _P(FePcgOpts),
                                                _P(_i64)]),
     'fe_pcg_batched_coarse': (_int, [_vp, _P(FeBsr), _P(FeBsr), _vp, _vp, _i32, _vp, _P(FeCoarse), _vp, _vp,

@@ -831,11 +831,11 @@ int finish_pcg(fe_handle* h, const Work& w, int nseg, fe_pcg_stats* s, const int
 // The solve by a team of workgroups in one launch (fe_pcg_team.h): one segment on the padded pattern, of
 // at most kTeamMaxTiles tiles.  Beyond that the launches are long enough that their latency no longer
 // matters (64^3 cube: 2,152 tiles, 31 us of its 64 us iteration in the row product) and the matrix would
-// not stay on the chip.  Sets *ran when it was launched and *done when the solve has
-// ended; otherwise x holds a starting point and the caller runs the launched kernels.
+// not stay on the chip.  Sets *path, and where that is not FE_PCG_ONE_LAUNCH x holds a starting point and the
+// caller runs the launched kernels.
 template <typename T, int D, int PC, int S, bool CO>
 int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
-             bool* ran, bool* done) {
+             int32_t* path) {
   const fe_bsr* A64 = pb.A64;
   const fe_bsr* Ait = pb.Ait;
   hipStream_t st = h->stream;
@@ -909,11 +909,10 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
     (void)hipGetLastError();  // this device or stream takes no cooperative launch
     return FE_OK;
   }
-  *ran = true;
   int32_t aborted = 0;
   int rc = finish_pcg(h, w, 1, s, a.abort, &aborted);
   if (rc) return rc;
-  *done = aborted == 0;
+  *path = aborted == 0 ? FE_PCG_ONE_LAUNCH : aborted == 1 ? FE_PCG_LEFT : FE_PCG_WIDE;
   return FE_OK;
 }
 
@@ -931,16 +930,16 @@ inline bool team_takes(int64_t n_rows, int dof, int elem, int64_t n_coarse) {
 
 template <typename T, int D, int PC, bool CO>
 int try_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
-             bool* ran, bool* done) {
+             int32_t* path) {
   const int64_t tiles = ceil_div(pb.A64->n_brows, tile_rows_dof(D));
   const int64_t nct = CO ? pb.C->n_agg * pb.C->nc : 0;
   if (!team_takes(pb.A64->n_brows, D, (int)sizeof(T), nct)) return FE_OK;
   // One workgroup per CU: the fewest threads per workgroup with which the chip holds the tiles, and up to
   // two tiles in one workgroup, whose messages stay in its LDS (40 x 10 plate, two tiles: 1.2 ms against
   // 2.3 ms by two workgroups).
-  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2, CO>(h, pb, w, o, s, ran, done);
-  if (tiles <= 256) return run_team<T, D, PC, 1, CO>(h, pb, w, o, s, ran, done);
-  if constexpr (sizeof(T) == 4 || (CO && D <= 2)) return run_team<T, D, PC, 4, CO>(h, pb, w, o, s, ran, done);
+  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2, CO>(h, pb, w, o, s, path);
+  if (tiles <= 256) return run_team<T, D, PC, 1, CO>(h, pb, w, o, s, path);
+  if constexpr (sizeof(T) == 4 || (CO && D <= 2)) return run_team<T, D, PC, 4, CO>(h, pb, w, o, s, path);
   return FE_OK;
 }
 
@@ -971,16 +970,14 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
   {
     int rc0 = launch_init();
     if (rc0) return rc0;
-    bool ran = false, done = false;
+    int32_t* path = &h->pcg_path;
     if (pb.ordered) {
-      if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, &ran, &done);
-      h->pcg_path = done ? FE_PCG_ONE_LAUNCH : ran ? FE_PCG_LEFT : FE_PCG_LAUNCHED;
-      return rc0 ? rc0 : done ? FE_OK : kErrTeamLeft;
+      if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, path);
+      return rc0 ? rc0 : *path == FE_PCG_ONE_LAUNCH ? FE_OK : kErrTeamLeft;
     }
-    if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, &ran, &done);
-    h->pcg_path = done ? FE_PCG_ONE_LAUNCH : ran ? FE_PCG_LEFT : FE_PCG_LAUNCHED;
-    if (rc0 || done) return rc0;
-    if (ran) rc0 = launch_init();  // the team gave up and left its state behind
+    if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, path);
+    if (rc0 || *path == FE_PCG_ONE_LAUNCH) return rc0;
+    if (*path != FE_PCG_LAUNCHED) rc0 = launch_init();  // the team gave up and left its state behind
     if (rc0) return rc0;
   }
   FE_CHECK_HIP(hipMemsetAsync(w.p, 0, n * sizeof(T), st));
@@ -1218,7 +1215,7 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
                int nseg, const int32_t* seg_nodes, const double* b, double* x, void* work,
                int64_t work_bytes, const fe_pcg_opts* o, fe_pcg_stats* s, fe_pcg_seg_stats* seg_out,
                const char* who, const fe_coarse* C = nullptr, const void* Ainv64 = nullptr,
-               const void* Ainv32 = nullptr, bool ordered = false) {
+               const void* Ainv32 = nullptr, bool ordered = false, bool finish = true) {
   const int elem = (int)sizeof(double);  // FP64-sized vectors: the FP64 fallback reuses them
   const int rows = tile_rows_dof(A64->dof);
   const int64_t ntiles = count_tiles(nseg, seg_nodes, rows);
@@ -1252,6 +1249,11 @@ int pcg_common(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M
                        : dispatch_dof<double>(h, pb, w, o, s);
   const int32_t path = h->pcg_path;  // (the solves below overwrite it)
   fe_pcg_opts o_plain = *o;
+  if (rc == kErrTeamLeft && !finish) {
+    FE_CHECK_HIP(hipStreamSynchronize(h->stream));  // the host tile arrays must outlive their copies
+    *s = fe_pcg_stats{};
+    return FE_OK;
+  }
   if (rc == kErrTeamLeft) {
     // the launched kernels finish an ordered solve in FP64, on A64 itself
     o_plain.mixed = 0;
@@ -1433,24 +1435,38 @@ extern "C" int fe_pcg_coarse_takes_ordered(const fe_bsr* A, const fe_coarse* C, 
   return FE_OK;
 }
 
-extern "C" int fe_pcg_coarse_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
-                                     const void* M32, const fe_coarse* C, const void* Ainv64, const double* b,
-                                     double* x, void* work, int64_t work_bytes, const fe_pcg_opts* o,
-                                     fe_pcg_stats* s) {
+static int pcg_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64, const void* M32,
+                       const fe_coarse* C, const void* Ainv64, const double* b, double* x, void* work,
+                       int64_t work_bytes, const fe_pcg_opts* o, fe_pcg_stats* s, const char* who, bool finish) {
   FE_ENTER(h);
-  FE_REQUIRE(b && x && work && o && s && C && A64 && Aord && M64 && Ainv64, "fe_pcg_coarse_ordered: null argument");
-  int rc = check_pcg_args(A64, Aord, M64, M32, o, "fe_pcg_coarse_ordered");
+  FE_REQUIRE(b && x && work && o && s && C && A64 && Aord && M64 && Ainv64, "%s: null argument", who);
+  int rc = check_pcg_args(A64, Aord, M64, M32, o, who);
   if (rc) return rc;
   int yes = 0;
   rc = fe_pcg_coarse_takes_ordered(A64, C, o, &yes);
   if (rc) return rc;
-  FE_REQUIRE(yes, "fe_pcg_coarse_ordered: not a system for the ordered form (fe_pcg_coarse_takes_ordered)");
-  FE_REQUIRE(Aord->row_align == 4, "fe_pcg_coarse_ordered: the iteration matrix must be on a padded pattern");
-  FE_REQUIRE(C->dof == A64->dof && C->n_nodes == A64->n_brows, "fe_pcg_coarse_ordered: coarse space and A disagree");
+  FE_REQUIRE(yes, "%s: not a system for the ordered form (fe_pcg_coarse_takes_ordered)", who);
+  FE_REQUIRE(Aord->row_align == 4, "%s: the iteration matrix must be on a padded pattern", who);
+  FE_REQUIRE(C->dof == A64->dof && C->n_nodes == A64->n_brows, "%s: coarse space and A disagree", who);
   *s = fe_pcg_stats{};
   const int32_t seg[2] = {0, (int32_t)A64->n_brows};
-  return pcg_common(h, A64, Aord, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr,
-                    "fe_pcg_coarse_ordered", C, Ainv64, nullptr, true);
+  return pcg_common(h, A64, Aord, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr, who, C, Ainv64, nullptr,
+                    true, finish);
+}
+
+extern "C" int fe_pcg_coarse_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
+                                     const void* M32, const fe_coarse* C, const void* Ainv64, const double* b,
+                                     double* x, void* work, int64_t work_bytes, const fe_pcg_opts* o,
+                                     fe_pcg_stats* s) {
+  return pcg_ordered(h, A64, Aord, M64, M32, C, Ainv64, b, x, work, work_bytes, o, s, "fe_pcg_coarse_ordered", true);
+}
+
+extern "C" int fe_pcg_coarse_one_launch(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
+                                        const void* M32, const fe_coarse* C, const void* Ainv64, const double* b,
+                                        double* x, void* work, int64_t work_bytes, const fe_pcg_opts* o,
+                                        fe_pcg_stats* s) {
+  return pcg_ordered(h, A64, Aord, M64, M32, C, Ainv64, b, x, work, work_bytes, o, s, "fe_pcg_coarse_one_launch",
+                     false);
 }
 
 extern "C" int fe_pcg_batched_coarse_workspace(fe_handle* h, const fe_bsr* A, int32_t n_seg,

@@ -150,6 +150,11 @@ __device__ inline int32_t team_here(int32_t v) {
   return v;
 }
 
+// Raise abort: 1 a wait reached its bound, 2 a workgroup's columns do not fit in its LDS (which stays 2).
+__device__ inline void team_give_up(int32_t* abort, int32_t why) {
+  __hip_atomic_fetch_max(abort, why, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Poll until `ready()`; false when another workgroup has given up or the bound is reached, which raises abort.
 template <typename F>
 __device__ inline bool team_poll(int32_t* abort, int32_t spins, F ready) {
@@ -157,7 +162,7 @@ __device__ inline bool team_poll(int32_t* abort, int32_t spins, F ready) {
     if (ready()) return true;
     if ((n & 63) == 63 && ld_team(abort) != 0) return false;
   }
-  st_team(abort, 1);
+  team_give_up(abort, 1);
   return false;
 }
 
@@ -993,7 +998,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       if (st.done || st.need_ru) break;
     }
   }
-  if (!alive && threadIdx.x == 0) st_team(a.abort, fits ? 1 : 2);
+  if (!alive && threadIdx.x == 0) team_give_up(a.abort, fits ? 1 : 2);
   // x is what the solve has reached, also after an aborted wait (the host continues from it)
 #pragma unroll
   for (int ps = 0; ps < kPasses; ++ps) {

@@ -444,6 +444,7 @@ class PaddedGraph:
         self.base = graph
         self.n_nodes = graph.n_nodes
         self.order = order
+        self.launched = set()  # precisions (mixed or not) that the one-launch solve does not take in this order
         if order is None:
             pptr, bcol, src = pad_pattern(graph.pattern.bptr, graph.pattern.bcol, a)
         else:
@@ -789,15 +790,16 @@ class PcgSolver:
         # the iteration matrix: a copy on the padded pattern (16-byte loads in the SpMV), FP32 with
         # mixed precision; A64 keeps the true residual
         # a two-level solve that fits on the chip takes it in the order of the aggregates
-        # (fe_pcg_coarse_ordered)
+        # (fe_pcg_coarse_one_launch)
         self.ordered = False
         if coarse is not None and segments is None and A32 is None:
             yes = ctypes.c_int()
             _hip.call('fe_pcg_coarse_takes_ordered', ctypes.byref(A64.struct()), ctypes.byref(coarse.struct()),
                       ctypes.byref(self._opts(1e-8, 1)), ctypes.byref(yes))
             self.ordered = bool(yes.value)
-        order = coarse.host.agg_nodes if self.ordered else None
-        self.A32 = A64.padded(torch.float32 if self.mixed else torch.float64, order) if A32 is None else A32
+            if self.ordered:
+                self.ordered = self.mixed not in ordered_graph(A64.graph, coarse.host.agg_nodes).launched
+        self.A32 = self._iteration_matrix(self.ordered) if A32 is None else A32
         self.M32 = _to_f32(self.ctx, self.M64) if self.mixed else None
         if coarse is not None:
             self.ctx.stream.wait_event(coarse_done)
@@ -822,6 +824,10 @@ class PcgSolver:
         return _hip.FePcgOpts(float(tol), int(max_iter), pc, int(self.mixed), int(self.check_every),
                               float(self.ru_delta), int(profile), int(self.graph))
 
+    def _iteration_matrix(self, ordered: bool):
+        return self.A64.padded(torch.float32 if self.mixed else torch.float64,
+                               self.coarse.host.agg_nodes if ordered else None)
+
     def _path(self):
         path = ctypes.c_int()
         _hip.call('fe_pcg_path', self.ctx.h, ctypes.byref(path))
@@ -830,9 +836,9 @@ class PcgSolver:
     def solve(self, b: torch.Tensor, x: Optional[torch.Tensor] = None, tol: float = 1e-8,
               max_iter: Optional[int] = None, profile: bool = False):
         """Solve from initial guess x (zeros if None); returns (x, info dict).  info['path'] tells how
-        it ran: ``FE_PCG_LAUNCHED`` kernels, ``FE_PCG_ONE_LAUNCH``, or ``FE_PCG_LEFT`` when the one
-        launch gave up and launched kernels finished.  With segments, info also holds per-segment
-        arrays (iterations, status, relres, ...)."""
+        it ran: ``FE_PCG_LAUNCHED`` kernels, ``FE_PCG_ONE_LAUNCH``, or ``FE_PCG_LEFT`` or
+        ``FE_PCG_WIDE`` when the one launch gave up and launched kernels finished.  With segments, info
+        also holds per-segment arrays (iterations, status, relres, ...)."""
         ctx = self.ctx
         if max_iter is None:
             max_iter = max(2000, min(10 * self.A64.n, 50000))
@@ -843,7 +849,7 @@ class PcgSolver:
         ordered = self.ordered and not profile
         it = self.A32
         if self.ordered and profile:  # the profiled kernels are the launched ones, in the mesh's order
-            it = self.A64.padded(torch.float32 if self.mixed else torch.float64)
+            it = self._iteration_matrix(False)
         a32 = it.struct() if it is not None else None
         nbytes = ctypes.c_int64()
         cstruct = self.coarse.struct() if self.coarse is not None else None
@@ -866,11 +872,22 @@ class PcgSolver:
             self._work = torch.empty(nbytes.value, dtype=torch.uint8, device=ctx.torch_device)
         stats = _hip.FePcgStats()
         a32p = ctypes.byref(a32) if a32 is not None else None
-        seg_info = None
+        seg_info = path = None
         if ordered:
-            _hip.call('fe_pcg_coarse_ordered', ctx.h, ctypes.byref(a64), a32p, _vp(self.M64), _vp(self.M32),
+            _hip.call('fe_pcg_coarse_one_launch', ctx.h, ctypes.byref(a64), a32p, _vp(self.M64), _vp(self.M32),
                       ctypes.byref(cstruct), _vp(self.Ainv64), _vp(b), _vp(x), _vp(self._work),
                       self._work.numel(), ctypes.byref(opts), ctypes.byref(stats))
+            path = self._path()
+            ordered = path == _hip.FE_PCG_ONE_LAUNCH
+            if not ordered:  # from the x it left, by the launched kernels in the same precision
+                it = self._iteration_matrix(False)
+                a32 = it.struct()
+                a32p = ctypes.byref(a32)
+                if path != _hip.FE_PCG_LEFT:  # nor will the launch take the system's next solve
+                    self.A32.graph.launched.add(self.mixed)
+                    self.A32, self.ordered = it, False
+        if ordered:
+            pass
         elif cstruct is not None and self.segments is None:
             _hip.call('fe_pcg_coarse', ctx.h, ctypes.byref(a64), a32p, _vp(self.M64), _vp(self.M32),
                       ctypes.byref(cstruct), _vp(self.Ainv64), _vp(self.Ainv32), _vp(b), _vp(x),
@@ -897,7 +914,7 @@ class PcgSolver:
                 'restarts': stats.restarts,
                 'status': stats.status, 'relres': stats.relres, 'relres_rec': stats.relres_rec,
                 'bnorm': stats.bnorm, 'spmv_ms': stats.spmv_ms, 'spmv_samples': stats.spmv_samples,
-                'fallbacks': stats.fallbacks, 'path': self._path()}
+                'fallbacks': stats.fallbacks, 'path': self._path() if path is None else path}
         if seg_info is not None:
             info['segments'] = seg_info
         return x, info

@@ -345,10 +345,13 @@ int fe_pcg(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64, 
 
 /* How the handle's last PCG solve (of any of these entry points) ran in the precision it began in:
    FE_PCG_LAUNCHED kernels for every step of every iteration, FE_PCG_ONE_LAUNCH all of it (a system that
-   fits on the chip), FE_PCG_LEFT begun in one launch, which gave up, and finished by launched kernels. */
+   fits on the chip), FE_PCG_LEFT begun in one launch, in which a wait reached its bound, and finished by
+   launched kernels, FE_PCG_WIDE likewise, but the launch ended before its first iteration because a
+   workgroup's columns do not fit in its LDS (a property of the pattern and its numbering). */
 #define FE_PCG_LAUNCHED 0
 #define FE_PCG_ONE_LAUNCH 1
 #define FE_PCG_LEFT 2
+#define FE_PCG_WIDE 3
 int fe_pcg_path(fe_handle* h, int* path);
 /* Bound of a wait between the workgroups of a one-launch solve, in polls of about a microsecond
    (FE_PCG_SPINS unless set).  A solve whose wait reaches it gives up and is finished by launched kernels;
@@ -467,6 +470,12 @@ int fe_pcg_coarse_takes_ordered(const fe_bsr* A, const fe_coarse* C, const fe_pc
 int fe_pcg_coarse_ordered(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
                           const void* M32, const fe_coarse* C, const void* Ainv64, const double* b, double* x,
                           void* work, int64_t work_bytes, const fe_pcg_opts* opts, fe_pcg_stats* stats);
+/* The same, for a caller that has (or makes) the matrix for fe_pcg_coarse too: a solve that the launch does
+   not end is not finished.  FE_OK with a path (fe_pcg_path) other than FE_PCG_ONE_LAUNCH: x holds a
+   starting point for fe_pcg_coarse, stats nothing. */
+int fe_pcg_coarse_one_launch(fe_handle* h, const fe_bsr* A64, const fe_bsr* Aord, const void* M64,
+                             const void* M32, const fe_coarse* C, const void* Ainv64, const double* b, double* x,
+                             void* work, int64_t work_bytes, const fe_pcg_opts* opts, fe_pcg_stats* stats);
 int fe_pcg_batched_coarse_workspace(fe_handle* h, const fe_bsr* A, int32_t n_seg, const int32_t* seg_nodes,
                                     const fe_coarse* C, const fe_pcg_opts* opts, int64_t* bytes);
 int fe_pcg_batched_coarse(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const void* M64,

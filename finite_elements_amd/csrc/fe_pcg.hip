@@ -26,6 +26,8 @@
 // One system small enough for the chip is solved in one launch instead (fe_pcg_team.h, with the same
 // arithmetic); the kernels here take larger systems, batches and profiled runs.
 #include <algorithm>
+#include <atomic>
+#include <optional>
 #include <vector>
 
 #include "fe_sparse.h"
@@ -828,6 +830,22 @@ int finish_pcg(fe_handle* h, const Work& w, int nseg, fe_pcg_stats* s, const int
   return FE_OK;
 }
 
+// Cooperative launches of a process take turns on a device, whatever their streams.  The solves that would use
+// one count themselves in, from there to their end.
+std::atomic<int> g_team_solves[64];
+struct TeamTurn {
+  std::atomic<int>* n;
+  int others;  // in flight when it came
+  explicit TeamTurn(int device) : n(&g_team_solves[device & 63]), others(n->fetch_add(1)) {}
+  TeamTurn(const TeamTurn&) = delete;
+  ~TeamTurn() { n->fetch_sub(1); }
+};
+// A solve that finds this many others runs by the launched kernels, to the same bits: these take two to three
+// turns alone, but overlap.  N 13^3 cubes (FP64 Jacobi) on N streams, in turns and launched: N = 2 6.7 and 15.1 ms,
+// 4 13.3 and 16.1, 8 27.0 and 18.1; 60^2 magnetostatics 2.5 and 3.4, 4.9 and 4.3, 10.0 and 7.4.  (The two-level
+// solve, six kernels per iteration when launched, is always faster in turns: eight 20^3 cubes 21.4 and 33.3 ms.)
+constexpr int kTeamOthers = 3;
+
 // The solve by a team of workgroups in one launch (fe_pcg_team.h): one segment on the padded pattern, of
 // at most kTeamMaxTiles tiles.  Beyond that the launches are long enough that their latency no longer
 // matters (64^3 cube: 2,152 tiles, 31 us of its 64 us iteration in the row product) and the matrix would
@@ -835,7 +853,7 @@ int finish_pcg(fe_handle* h, const Work& w, int nseg, fe_pcg_stats* s, const int
 // caller runs the launched kernels.
 template <typename T, int D, int PC, int S, bool CO>
 int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
-             int32_t* path) {
+             int32_t* path, std::optional<TeamTurn>* turn) {
   const fe_bsr* A64 = pb.A64;
   const fe_bsr* Ait = pb.Ait;
   hipStream_t st = h->stream;
@@ -897,6 +915,11 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   FE_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   FE_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock * S, (size_t)lds));
   if (grid > (int64_t)per_cu * h->num_cus) return FE_OK;
+  // one workgroup waits for no other: an ordinary launch, beside those of other streams
+  if (grid > 1) {
+    turn->emplace(h->device);
+    if (!CO && (*turn)->others >= kTeamOthers) return FE_OK;
+  }
   FE_CHECK_HIP(hipMemsetAsync(w.flags, 0, (kTeamMaxTiles + 1) * sizeof(uint64_t), st));
   if constexpr (CO && sizeof(T) == 4) {
     const int64_t n = pb.C->n_agg * NC * a.lda;
@@ -904,10 +927,14 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
                        w.ainv32);
   }
   void* args[] = {&a};
-  hipError_t e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)grid), dim3(kBlock * S), args, (unsigned)lds, st);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();  // this device or stream takes no cooperative launch
-    return FE_OK;
+  const dim3 wgs((unsigned)grid), threads(kBlock * S);
+  if (grid > 1) {
+    if (hipLaunchCooperativeKernel(kernel, wgs, threads, args, (unsigned)lds, st) != hipSuccess) {
+      (void)hipGetLastError();  // this device or stream takes no cooperative launch
+      return FE_OK;
+    }
+  } else {
+    FE_CHECK_HIP(hipLaunchKernel(kernel, wgs, threads, args, (size_t)lds, st));
   }
   int32_t aborted = 0;
   int rc = finish_pcg(h, w, 1, s, a.abort, &aborted);
@@ -930,16 +957,16 @@ inline bool team_takes(int64_t n_rows, int dof, int elem, int64_t n_coarse) {
 
 template <typename T, int D, int PC, bool CO>
 int try_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o, fe_pcg_stats* s,
-             int32_t* path) {
+             int32_t* path, std::optional<TeamTurn>* turn) {
   const int64_t tiles = ceil_div(pb.A64->n_brows, tile_rows_dof(D));
   const int64_t nct = CO ? pb.C->n_agg * pb.C->nc : 0;
   if (!team_takes(pb.A64->n_brows, D, (int)sizeof(T), nct)) return FE_OK;
   // One workgroup per CU: the fewest threads per workgroup with which the chip holds the tiles, and up to
   // two tiles in one workgroup, whose messages stay in its LDS (40 x 10 plate, two tiles: 1.2 ms against
   // 2.3 ms by two workgroups).
-  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2, CO>(h, pb, w, o, s, path);
-  if (tiles <= 256) return run_team<T, D, PC, 1, CO>(h, pb, w, o, s, path);
-  if constexpr (sizeof(T) == 4 || (CO && D <= 2)) return run_team<T, D, PC, 4, CO>(h, pb, w, o, s, path);
+  if (tiles == 2 || (tiles > 256 && tiles <= 512)) return run_team<T, D, PC, 2, CO>(h, pb, w, o, s, path, turn);
+  if (tiles <= 256) return run_team<T, D, PC, 1, CO>(h, pb, w, o, s, path, turn);
+  if constexpr (sizeof(T) == 4 || (CO && D <= 2)) return run_team<T, D, PC, 4, CO>(h, pb, w, o, s, path, turn);
   return FE_OK;
 }
 
@@ -959,7 +986,7 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
   hipStream_t st = h->stream;
   const T* M = (const T*)pb.M;
   const dim3 gt((unsigned)nt), gseg((unsigned)nseg);
-  h->pcg_path = FE_PCG_LAUNCHED;
+  std::optional<TeamTurn> turn;
   auto launch_init = [&]() -> int {
     hipLaunchKernelGGL((k_tile_norm<D>), gt, dim3(kBlock), 0, st, w.tiles, pb.b, w.partials);
     hipLaunchKernelGGL(k_pcg_init, gseg, dim3(kRed), 0, st, w.seg_tiles, nt, w.partials, w.st, o->tol,
@@ -971,11 +998,12 @@ int run_pcg(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* o
     int rc0 = launch_init();
     if (rc0) return rc0;
     int32_t* path = &h->pcg_path;
+    *path = FE_PCG_LAUNCHED;
     if (pb.ordered) {
-      if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, path);
+      if constexpr (PC == FE_PC_BLOCK_JACOBI) rc0 = try_team<T, D, PC, true>(h, pb, w, o, s, path, &turn);
       return rc0 ? rc0 : *path == FE_PCG_ONE_LAUNCH ? FE_OK : kErrTeamLeft;
     }
-    if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, path);
+    if (nseg == 1 && !pb.C && !o->profile && vec) rc0 = try_team<T, D, PC, false>(h, pb, w, o, s, path, &turn);
     if (rc0 || *path == FE_PCG_ONE_LAUNCH) return rc0;
     if (*path != FE_PCG_LAUNCHED) rc0 = launch_init();  // the team gave up and left its state behind
     if (rc0) return rc0;

@@ -106,7 +106,8 @@ def upload(ctx, *arrays):
         dev = ctx.tensor(host)
         for k, off in zip(small, starts):
             a = arrays[k]
-            out[k] = dev[int(off):int(off) + a.nbytes].view(torch.as_tensor(a).dtype).reshape(a.shape)
+            # .data: a tensor of its own for autograd (views of one tensor share the count of in-place changes)
+            out[k] = dev[int(off):int(off) + a.nbytes].view(torch.as_tensor(a).dtype).reshape(a.shape).data
     return out
 
 

@@ -135,9 +135,12 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid(LobParams p, const doubl
 // --------------------------------------------------------------------------------------------------
 // K1 and K1b's restriction in one pass (two-level preconditioner): chunk b of the residual partials
 // takes aggregates [b n_agg / chunks, (b+1) n_agg / chunks), or part b % agg_parts of aggregate b / agg_parts,
-// and walks their nodes (every node lies in one aggregate), forming R, W = T R and the column norms as k_lob_resid does and r_c = P^T R (thread
-// (group g, column j) sums an aggregate's nodes g, g + npg, ..., then the groups are added in a
-// fixed order), so K X and M X are read once per iteration.
+// and walks their nodes (every node lies in one aggregate), forming R, W = T R and the column norms as
+// k_lob_resid does and r_c = P^T R (thread (group g, column j) sums an aggregate's nodes g, g + npg, ...,
+// then the groups are added in a fixed order), so K X and M X are read once per iteration.  A soft-locked
+// column has no part of W, the coarse one included: with the coarse parts of more locked columns than there are
+// coarse modes, or of nearly equal pairs, W's columns depend on each other, and every iteration restarts
+// without P (8 pairs to 1e-7 on a 6^3 cube: 474 to 1,999 iterations, 85 to 97 without those parts).
 template <int D, int NC>
 __global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coarse C, int64_t ld,
                                                             const double* __restrict__ T, int64_t t_stride,
@@ -193,8 +196,9 @@ __global__ __launch_bounds__(kThreads) void k_lob_resid_agg(LobParams p, fe_coar
           rr += R[e] * R[e];
           bb += mx * mx;
           const double* Pr = C.P + (i * D + e) * NC;
+          const double rl = s_lock[j] ? 0.0 : R[e];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) acc[c] += Pr[c] * R[e];
+          for (int c = 0; c < NC; ++c) acc[c] += Pr[c] * rl;
         }
 #pragma unroll
         for (int e = 0; e < D; ++e) {

@@ -1,0 +1,35 @@
+"""Soft-locked pairs leave the search to the others: a looser tolerance locks pairs earlier and needs no more
+iterations for it, and a block without guard vectors converges to its last pair."""
+
+import pytest
+
+from finite_elements_amd import device, modal
+from tests.test_gpu_modal import _check_pairs, _modal_system, _oracle_pencil, eigen
+
+pytestmark = pytest.mark.gpu
+
+
+def _pencil(n, seed):
+    pr, s = _modal_system(n, seed)
+    fixed, _ = s.dirichlet(pr.fixed_dofs)
+    KD = device.apply_dirichlet(s.stiffness_bsr(), fixed)
+    MD = device.apply_dirichlet(s.mass_bsr(), fixed)
+    return pr, s, fixed, KD, MD
+
+
+@pytest.mark.parametrize('n', [6, 9, 12])
+def test_two_level_iterations_by_tolerance(ctx, n):
+    print(f'two-level by tolerance {n}', flush=True)
+    pr, s, fixed, KD, MD = _pencil(n, 5000)
+    coarse = s.coarse_space(pr.fixed_dofs)
+    Ko, Mo = _oracle_pencil(pr)
+    ref, _ = eigen.smallest_clamped(Ko, Mo, pr.fixed_dofs, 8)
+    for seed in range(4):
+        its = []
+        for tol in (1e-5, 1e-7, 1e-9):
+            vals, vecs, info = modal.lobpcg(KD, MD, 8, fixed=fixed, tol=tol, max_iter=3000, coarse=coarse, seed=seed)
+            assert info['status'] == 0
+            its.append(int(info['iterations'][0]))
+        _check_pairs(vals[0], vecs[0].cpu().numpy(), Ko, Mo, pr.fixed_dofs, ref)
+        # two decades of the residual are some tens of iterations: a tenth of them is the scatter
+        assert its[0] <= its[1] * 1.1 and its[1] <= its[2] * 1.1, its

@@ -1064,10 +1064,10 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   const int v = blockIdx.x;
   LobState* s = st + v;
   __shared__ int s_skip, s_ns, s_init, s_keep;
-  __shared__ int s_kept[kMaxBasis];
+  __shared__ int s_kept[kMaxBasis], s_ord[kMaxBasis];
   __shared__ int s_sel[kMaxBlock];
   __shared__ double s_scale[kMaxBasis];
-  __shared__ double s_mu[kMaxBasis];
+  __shared__ double s_piv[kMaxBasis], s_mu[kMaxBasis];
   __shared__ double s_norm[2 * kMaxBlock];
   const int m = p.m, NS = 3 * m, tid = threadIdx.x;
   if (tid == 0) {
@@ -1119,25 +1119,58 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   const double* GM = GK + NS * NS;
   double* Z = Zg + (int64_t)v * NS * NS;
   // ---- M-orthonormalisation of the basis with a rank check: Cholesky of D GM D, D = diag(GM)^-1/2, in the
-  // order X, W, P, dropping a column whose pivot (the squared norm of what its predecessors leave of it)
-  // is at most p.drop.  sA holds the Schur complement, sV the basis change Z: step k takes column k
-  // out of the columns after it, in both.  One barrier per step; the eigen-decomposition that this replaces
-  // took eight to ten sweeps of steps (354 us at r = 36).
+  // order s_ord: X, W, P's columns of active pairs, then those of soft-locked ones (W column zero).  sA holds the
+  // Schur complement, sV the basis change Z: step k takes column k out of the columns after it, in both.
+  // A column is dropped when its pivot (the squared norm of what its predecessors leave of it) is at most
+  // p.drop of the squared norm of its column of Z: their quotient is a Rayleigh quotient of the scaled Gram
+  // matrix and bounds its smallest eigenvalue.
+  // The P of many locked pairs are built from the W of the few active ones and come to depend on each other
+  // and on the active pairs' P: these stay ahead of them, and dropping one of them does not restart the search.
+  // (In the order of the pairs, an active P was the one dropped, and what was left was steepest descent:
+  // 8 pairs in blocks of 8 to 1e-9 on 9^3 to 16^3 cubes did not converge in 3,000 iterations in 20 of 96
+  // runs; now 1, and 7 with the eigenvalue test.)  One barrier per step; the eigen-decomposition that this
+  // replaces took eight to ten sweeps of steps (354 us at r = 36).
   if (tid < ns) {
     const double d = GM[tid * NS + tid];
     s_scale[tid] = d > 0.0 ? 1.0 / sqrt(d) : 0.0;
   }
   __syncthreads();
+  if (tid < ns) {
+    int at = tid;
+    if (tid >= 2 * m) {
+      int before = 0, active = 0;  // of P's active columns
+      for (int j = 0; j < m; ++j) {
+        const bool on = s_scale[m + j] > 0.0;
+        active += on;
+        before += on && j < tid - 2 * m;
+      }
+      at = s_scale[tid - m] > 0.0 ? 2 * m + before : tid + active - before;
+    }
+    s_ord[at] = tid;
+  }
+  __syncthreads();
   const int wave = tid >> 6, nwaves = blockDim.x >> 6, lane = tid & 63;
   for (int a = wave; a < ns; a += nwaves)
     for (int b = lane; b < ns; b += 64) {
-      sA[a * ns + b] = 0.5 * (GM[a * NS + b] + GM[b * NS + a]) * s_scale[a] * s_scale[b];
+      const int ga = s_ord[a], gb = s_ord[b];
+      sA[a * ns + b] = 0.5 * (GM[ga * NS + gb] + GM[gb * NS + ga]) * s_scale[ga] * s_scale[gb];
       sV[a * ns + b] = a == b ? 1.0 : 0.0;
     }
   __syncthreads();
+  bool near = false;
   for (int k = 0; k < ns; ++k) {
     const double piv = sA[k * ns + k];
-    if (piv > p.drop) {  // uniform
+    near = near || !(piv > 1e-4);
+    double vv = 1.0;
+    if (near) {  // with larger pivots alone a column of Z stays small: its norm is not formed
+      vv = 0.0;
+      for (int i = lane; i <= k; i += 64) vv += sV[i * ns + k] * sV[i * ns + k];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) vv += __shfl_xor(vv, o, 64);
+    }
+    const bool keep = piv > p.drop * vv;  // uniform
+    if (tid == 0) s_piv[k] = keep ? piv : 0.0;
+    if (keep) {
       const double inv = 1.0 / piv;
       for (int j = k + 1 + lane; j < ns; j += 64) {
         const double f = sA[k * ns + j] * inv;
@@ -1150,9 +1183,11 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
   if (tid == 0) {
     int kept = 0, zero = 0;
     for (int k = 0; k < ns; ++k) {
-      const double mu = sA[k * ns + k];
-      zero += !(s_scale[k] > 0.0);
-      if (mu > p.drop) {
+      const double mu = s_piv[k];
+      const int g = s_ord[k];
+      const bool locked = g >= 2 * m && !(s_scale[g - m] > 0.0);
+      zero += !(s_scale[g] > 0.0) || (locked && !(mu > 0.0));
+      if (mu > 0.0) {
         s_kept[kept] = k;
         s_mu[kept] = mu;
         ++kept;
@@ -1160,7 +1195,7 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
     }
     s_keep = kept;
     s->kept = kept;
-    // directions dropped for near-dependence (soft-locked W columns aside): the next iteration
+    // directions dropped for near-dependence (soft-locked pairs' columns aside): the next iteration
     // restarts the search from [X W] without P
     s->restart = (kept + zero < ns);
   }
@@ -1178,14 +1213,17 @@ __global__ __launch_bounds__(kRRThreads) void k_lob_rr(LobParams p, LobState* st
       const int idx = tid + t * kRRThreads;
       if (idx < ns * rk) {
         const int a = idx / rk, k = idx - a * rk;
-        z[t] = s_scale[a] * sV[a * ns + s_kept[k]] / sqrt(s_mu[k]);
-        Z[a * NS + k] = z[t];
+        z[t] = s_scale[s_ord[a]] * sV[a * ns + s_kept[k]] / sqrt(s_mu[k]);
+        Z[s_ord[a] * NS + k] = z[t];
       }
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < kRRItems; ++t)
-      if (tid + t * kRRThreads < ns * rk) sV[tid + t * kRRThreads] = z[t];
+      if (tid + t * kRRThreads < ns * rk) {
+        const int a = (tid + t * kRRThreads) / rk;
+        sV[tid + t * kRRThreads + (s_ord[a] - a) * rk] = z[t];
+      }
   }
   for (int a = wave; a < ns; a += nwaves)
     for (int b = lane; b < ns; b += 64) sA[a * ns + b] = 0.5 * (GK[a * NS + b] + GK[b * NS + a]);

@@ -33,3 +33,14 @@ def test_two_level_iterations_by_tolerance(ctx, n):
         _check_pairs(vals[0], vecs[0].cpu().numpy(), Ko, Mo, pr.fixed_dofs, ref)
         # two decades of the residual are some tens of iterations: a tenth of them is the scatter
         assert its[0] <= its[1] * 1.1 and its[1] <= its[2] * 1.1, its
+
+
+@pytest.mark.parametrize('seed', range(16))
+def test_block_without_guard_vectors(ctx, seed):
+    print(f'no guard vectors {seed}', flush=True)
+    pr, s, fixed, KD, MD = _pencil(12, 5000)
+    vals, _, info = modal.lobpcg(KD, MD, 8, block=8, fixed=fixed, tol=1e-9, max_iter=3000, seed=seed)
+    assert info['status'] == 0, info['resid']
+    Ko, Mo = _oracle_pencil(pr)
+    ref, _ = eigen.smallest_clamped(Ko, Mo, pr.fixed_dofs, 8)
+    assert abs(vals[0] / ref - 1).max() < 1e-8

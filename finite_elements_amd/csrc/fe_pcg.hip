@@ -912,7 +912,8 @@ int run_team(fe_handle* h, const Problem& pb, const Work& w, const fe_pcg_opts* 
   const void* kernel = (const void*)k_pcg_team<T, D, PC, S, CO>;
   const int64_t grid = ceil_div(a.ntiles, S);
   int per_cu = 0;
-  FE_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // the same bound for every system: another thread may set it between this call and the launch
+  FE_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kTeamLds));
   FE_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock * S, (size_t)lds));
   if (grid > (int64_t)per_cu * h->num_cus) return FE_OK;
   // one workgroup waits for no other: an ordinary launch, beside those of other streams

@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kBlock) void k_gnn_layer_wgrad(int64_t nb, const fl
       const float delta = hv[u] > 0.f ? dv[u] : 0.f;
       db += delta;
       acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(delta, x[u], acc[0], 0, 0, 0);
-      if (FIN == GW) acc[FIN == GW ? 1 : 0] = __builtin_amdgcn_mfma_f32_32x32x2f32(delta, y[u], acc[FIN == GW ? 1 : 0], 0, 0, 0);
+      if constexpr (FIN == GW) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(delta, y[u], acc[1], 0, 0, 0);
     }
   }
   // accumulator register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32

@@ -15,9 +15,9 @@
 // two of three trips to memory of about 0.8 us (the wait for the data's stores, and the load after the
 // flag).  The reliable updates (a few per solve) use flags.  The matrix, or where it is too wide its
 // columns, stays in registers for the whole solve; vectors are in registers between updates.
-// Per iteration, launched kernels and this: 40 x 10 plate FP64 (one workgroup) 11.2 -> 3.2 us, 13^3 cube
-// FP64 (22 workgroups) 17 -> 6.2 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.2 us; two-level mixed 27^3 cube
-// (172) 40 -> 14 us, 450^2 magnetostatics (199) 33 -> 13 us.
+// Per iteration, launched kernels and this: 40 x 10 plate FP64 (one workgroup) 11.2 -> 2.8 us, 13^3 cube
+// FP64 (22 workgroups) 17 -> 7.4 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.3 us; two-level mixed 27^3 cube
+// with shuffled nodes (172) 40 -> 14.2 us, 450^2 magnetostatics (199) 33 -> 12.6 us.
 //
 // Two-level preconditioner (CO): the node rows are numbered aggregate by aggregate (order), so that a
 // workgroup's rows touch few aggregates.  The correction P A_c^-1 P^T r is carried by the recurrence of r:
@@ -42,7 +42,8 @@
 // chunk ends -- is that of the launched kernels (fe_pcg.hip), so a system solved here without a
 // coarse correction has the bits of the same system solved as a segment of a batch.
 //
-// The launch is cooperative (all workgroups resident, cooperative launches never side by side).  Every
+// The launch of more than one workgroup is cooperative (all of them resident; a process' cooperative launches on
+// a device take turns).  Every
 // wait is bounded: a thread that has polled `spins` times raises `abort`, which ends every other wait, its own
 // next ones and the other workgroups', after 64 polls; a workgroup leaves at the end of the meeting, and the
 // host finishes the solve with the launched kernels.
@@ -470,13 +471,9 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
       return t;
     };
     if (alone) {
-      // the butterfly over one to four tiles and zeros, written out
+      // the butterfly over one or two tiles and zeros, written out (four are in one of many workgroups)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        if constexpr (S == 1) v[k] = tile_sum(0, k);
-        if constexpr (S == 2) v[k] = tile_sum(0, k) + tile_sum(1, k);
-        if constexpr (S == 4) v[k] = (tile_sum(0, k) + tile_sum(2 % S, k)) + (tile_sum(1 % S, k) + tile_sum(3 % S, k));
-      }
+      for (int k = 0; k < 3; ++k) v[k] = S == 1 ? tile_sum(0, k) : tile_sum(0, k) + tile_sum(S - 1, k);
       return true;
     }
     uint64_t* box = a.pt + (int64_t)(tag & 1) * (6 * kTeamCopies) * a.pstride;

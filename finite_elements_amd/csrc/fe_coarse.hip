@@ -524,7 +524,8 @@ __global__ __launch_bounds__(kSegThreads) void k_coarse_inv_seg(fe_coarse C, dou
 }
 
 // The inverse (in src, which may be A) symmetrised into A (average with its transpose) with its FP32 copy.  A
-// workgroup takes a 32 x 32 tile and its mirror image, through LDS so that both are read and written by rows (1,280 x 1,280: 25 us without, 7 with).
+// workgroup takes a 32 x 32 tile and its mirror image, through LDS so that both are read and written by rows
+// (1,280 x 1,280: 25 us without, 7 with).
 constexpr int kSymTile = 32;
 __global__ __launch_bounds__(256) void k_sym_cast(int64_t n, int64_t ld, const double* src, double* A,
                                                   float* __restrict__ A32) {
@@ -655,8 +656,9 @@ __global__ __launch_bounds__(256) void k_coarse_gemv(int64_t n, int64_t ld, cons
 
 // Block-diagonal space: z_s = A_s^-1 r_s, one workgroup per segment; the threads (way, i) form row i from column
 // i of the symmetric block (coalesced over i), way taking entries way, way + kSegWays, ..., and the ways
-// are added in order.  Bound by the latency of a row's loads (256 plates: 8.7 us
-// with one way, 5.5 with eight).  The blocks are read in FP64 at every precision: a thin mesh's coarse block is too ill-conditioned for an FP32 inverse.
+// are added in order.  Bound by the latency of a row's loads (256 plates: 8.7 us with one way, 5.5 with eight).
+// The blocks are read in FP64 at every precision: a thin mesh's coarse block is too ill-conditioned for an
+// FP32 inverse.
 constexpr int kSegWays = 8;
 template <typename T>
 __global__ __launch_bounds__(kSegMax * kSegWays) void k_coarse_gemv_seg(fe_coarse C, const double* __restrict__ Ainv,

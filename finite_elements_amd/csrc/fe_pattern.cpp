@@ -360,10 +360,11 @@ extern "C" int fe_pattern_create(const int32_t* conn, int npe, int dof, int64_t 
     if (rc == FE_OK) {
       // default row-block schedule: 192 (tets) / 128 (triangles) incidences per workgroup, or one per
       // thread (256) where that still gives each of the 256 CUs eight ranges, raised to the largest node
-      // incidence count when a node has more (dynamic LDS stays under 64 KB for typical meshes: 36 doubles per
-      // tet incidence).  Longer ranges share more of their elements: 64^3 cube 237 -> 211 us, 450^2
-      // magnetostatics 39 -> 27, 700 x 350 plate 46 -> 32 (shuffled 76 -> 74); near 400,000 incidences a mass
-      // matrix loses 3% (26^3 cube 13.9 -> 14.4 us), so the line lies above that.
+      // incidence count when a node has more (a workgroup's LDS holds a record of up to 15 doubles per element
+      // of its range, at most one per incidence, and the range's maps: 256 tet incidences 30 KB and 7).
+      // Longer ranges share more of their elements: 64^3 cube 237 -> 211 us, 450^2 magnetostatics 39 -> 27,
+      // 700 x 350 plate 46 -> 32 (shuffled 76 -> 74); near 400,000 incidences a mass matrix loses 3% (26^3 cube
+      // 13.9 -> 14.4 us), so the line lies above that.
       int32_t cap = npe == 4 ? 192 : 128;
       if (p->inc_ptr[n_nodes] >= 8 * 256 * 256) cap = 256;
       for (int64_t i = 0; i < n_nodes; ++i) cap = std::max(cap, p->inc_ptr[i + 1] - p->inc_ptr[i]);

@@ -741,7 +741,8 @@ class PcgSolver:
 
     ``segments``: node-row offsets (n_seg + 1 entries) of independent blocks of a block-diagonal
     system (e.g. many plates assembled together); each block then iterates and stops on its own
-    (``fe_pcg_batched``).  ``graph``: replay each chunk of iterations from a captured HIP graph.
+    (``fe_pcg_batched``).  ``graph``: replay each chunk of iterations from a captured HIP graph (of
+    the launched kernels: a system that is solved in one launch, ``info['path']``, has no chunks).
     ``M64``: block preconditioner [n_nodes][d][d] FP64, a callable returning it, or None (the blocks
     of A64)."""
 

@@ -161,7 +161,8 @@ typedef struct {
   double ru_delta;       /* mixed: reliable update when ||r|| fell by this factor since the last one */
   int32_t profile;       /* 1: after the solve, time 20 back-to-back launches of the iteration's
                             SpMV kernel on the final state with HIP events (stats->spmv_ms) */
-  int32_t graph;         /* 1: capture one chunk of iterations in a HIP graph and replay it */
+  int32_t graph;         /* 1: capture one chunk of iterations in a HIP graph and replay it (launched
+                            kernels only: a solve in one launch, fe_pcg_path, has no chunks to replay) */
 } fe_pcg_opts;
 
 typedef struct {

@@ -1390,6 +1390,7 @@ extern "C" int fe_pcg(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32, const 
   if (rc) return rc;
   FE_REQUIRE(A64->n_brows < ((int64_t)1 << 31), "fe_pcg: too many node rows");
   *s = fe_pcg_stats{};
+  h->pcg_path = FE_PCG_LAUNCHED;
   if (A64->n_brows == 0) return FE_OK;
   const int32_t seg[2] = {0, (int32_t)A64->n_brows};
   return pcg_common(h, A64, A32, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr, "fe_pcg");
@@ -1449,6 +1450,7 @@ extern "C" int fe_pcg_coarse(fe_handle* h, const fe_bsr* A64, const fe_bsr* A32,
              "fe_pcg_coarse: missing coarse inverse (FP32 inverse and P32 for mixed precision)");
   FE_REQUIRE(A64->n_brows < ((int64_t)1 << 31), "fe_pcg_coarse: too many node rows");
   *s = fe_pcg_stats{};
+  h->pcg_path = FE_PCG_LAUNCHED;
   if (A64->n_brows == 0) return FE_OK;
   const int32_t seg[2] = {0, (int32_t)A64->n_brows};
   return pcg_common(h, A64, A32, M64, M32, 1, seg, b, x, work, work_bytes, o, s, nullptr,

@@ -2,6 +2,8 @@
 sizes, against the launched kernels (bit for bit without a coarse space; with one, the correction is
 carried by recurrence, so by tolerance and iterations)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -89,3 +91,17 @@ def test_two_level_limits(ctx, kind, size, shuffled, precision):
     _, launched = solver.solve(b, tol=tol, profile=True)
     assert launched['path'] == LAUNCHED and launched['status'] == 0
     assert abs(info['iterations'] - launched['iterations']) <= 16 + launched['iterations'] // 8
+
+
+def test_empty_system(ctx):
+    """A system without rows launches nothing, whatever ran before it."""
+    s, KD, b, _ = _prepared(ctx, 'tri_elastic', (5, 2))
+    solver = s.solver(KD, 'jacobi', 'fp64')
+    assert solver.solve(b, tol=1e-9)[1]['path'] == ONE_LAUNCH
+    empty = KD.struct()
+    empty.n_brows = empty.nnzb = 0
+    opts, stats, p = solver._opts(1e-9, 10), _hip.FePcgStats(), device._vp
+    work = torch.empty(4096, dtype=torch.uint8, device=b.device)
+    _hip.call('fe_pcg', ctx.h, ctypes.byref(empty), None, p(solver.M64), None, p(b), p(torch.zeros_like(b)), p(work),
+              work.numel(), ctypes.byref(opts), ctypes.byref(stats))
+    assert stats.status == 0 and solver._path() == LAUNCHED

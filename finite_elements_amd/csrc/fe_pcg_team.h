@@ -48,9 +48,9 @@
 //
 // The launch of more than one workgroup is cooperative (all of them resident; a process' cooperative launches on
 // a device take turns).  Every
-// wait is bounded: a thread that has polled `spins` times raises `abort`, which ends every other wait, its own
-// next ones and the other workgroups', after 64 polls; a workgroup leaves at the end of the meeting, and the
-// host finishes the solve with the launched kernels.
+// wait is bounded: a thread that has polled `spins` times notes it for its workgroup, whose waits, its own next
+// ones among them, then end after 64 polls; the workgroup leaves at the end of the meeting and raises `abort`,
+// which the others' waits look at as often, and the host finishes the solve with the launched kernels.
 #pragma once
 
 #include "fe_sparse.h"
@@ -161,14 +161,15 @@ __device__ inline void team_give_up(int32_t* abort, int32_t why) {
   __hip_atomic_fetch_max(abort, why, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Poll until `ready()`; false when another workgroup has given up or the bound is reached, which raises abort.
+// Poll until `ready()`; false, noted in *fail, when the bound is reached or this or another workgroup has given
+// up.  (Raising abort here as well costs registers at every poll: the four-tile kernels spilled twice as many.)
 template <typename F>
-__device__ inline bool team_poll(int32_t* abort, int32_t spins, F ready) {
+__device__ inline bool team_poll(const int32_t* abort, int32_t spins, int* fail, F ready) {
   for (int32_t n = 0; n < spins; ++n) {
     if (ready()) return true;
-    if ((n & 63) == 63 && ld_team(abort) != 0) return false;
+    if ((n & 63) == 63 && (ld_team(abort) != 0 || *(volatile int*)fail)) break;
   }
-  team_give_up(abort, 1);
+  *(volatile int*)fail = 1;
   return false;
 }
 
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
   auto meet_neighbours = [&]() {
     arrive();
     for (int g = lo + (int)threadIdx.x; g <= hi; g += NT)
-      if (!team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
+      team_poll(a.abort, a.spins, &s_fail, [&] { return ld_team(a.flags + g) >= epoch; });
     __syncthreads();
     return s_fail == 0;
   };
@@ -393,10 +394,8 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = 0.0;
     if (sub == 0) {
-      bool ok = true;
       for (int t = tid; t < a.ntiles; t += kBlock)
-        ok = ok && team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + t / S) >= epoch; });
-      if (!ok) s_fail = 1;
+        team_poll(a.abort, a.spins, &s_fail, [&] { return ld_team(a.flags + t / S) >= epoch; });
       // at most S kBlock tiles: one per workgroup of S subgroups, one workgroup per CU
       double e[S][NV];
 #pragma unroll
@@ -452,12 +451,11 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
       for (int j = 0; j < B; ++j) {
         if (e0 + j * NT >= nr * D) break;
-        if (!team_got(m[j], TW, tag) && !team_poll(a.abort, a.spins, [&] {
+        if (!team_got(m[j], TW, tag)) team_poll(a.abort, a.spins, &s_fail, [&] {
 #pragma unroll
-              for (int h = 0; h < TW; ++h) m[j][h] = ld_team(from[j] + h);
-              return team_got(m[j], TW, tag);
-            }))
-          s_fail = 1;
+          for (int h = 0; h < TW; ++h) m[j][h] = ld_team(from[j] + h);
+          return team_got(m[j], TW, tag);
+        });
         ul[S * R * D + e0 + j * NT] = team_value(m[j]);
       }
     }
@@ -503,7 +501,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
 #pragma unroll
       for (int j = 0; j < S; ++j) {
         if (tid + j * kBlock >= a.ntiles) break;
-        if (!got(j) && !team_poll(a.abort, a.spins, [&] { load(j); return got(j); })) s_fail = 1;
+        if (!got(j)) team_poll(a.abort, a.spins, &s_fail, [&] { load(j); return got(j); });
 #pragma unroll
         for (int k = 0; k < 3; ++k) v[k] += team_value(m[j][k]);
       }
@@ -689,7 +687,7 @@ __global__ __launch_bounds__(kBlock* S) void k_pcg_team(TeamArgs a) {
     } else {
       arrive();
       for (int g = threadIdx.x; g < nwg; g += NT)
-        if (!team_poll(a.abort, a.spins, [&] { return ld_team(a.flags + g) >= epoch; })) s_fail = 1;
+        team_poll(a.abort, a.spins, &s_fail, [&] { return ld_team(a.flags + g) >= epoch; });
       __syncthreads();
       if (turn == 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the ring's first region, also the first time
     }

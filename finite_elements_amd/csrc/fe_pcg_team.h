@@ -16,8 +16,8 @@
 // flag).  The reliable updates (a few per solve) use flags.  The matrix, or where it is too wide its
 // columns, stays in registers for the whole solve; vectors are in registers between updates.
 // Per iteration, launched kernels and this: 40 x 10 plate FP64 (one workgroup) 11.2 -> 2.8 us, 13^3 cube
-// FP64 (22 workgroups) 17 -> 7.4 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.3 us; two-level mixed 27^3 cube
-// with shuffled nodes (172) 40 -> 14.2 us, 450^2 magnetostatics (199) 33 -> 12.6 us.
+// FP64 (22 workgroups) 17 -> 6.6 us, 150^2 magnetostatics FP64 (90) 13.6 -> 5.4 us; two-level mixed 27^3 cube
+// with shuffled nodes (172) 40 -> 14.3 us, 450^2 magnetostatics (199) 33 -> 12.7 us.
 //
 // Two-level preconditioner (CO): the node rows are numbered aggregate by aggregate (order), so that a
 // workgroup's rows touch few aggregates.  The correction P A_c^-1 P^T r is carried by the recurrence of r:
